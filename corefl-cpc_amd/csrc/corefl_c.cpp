@@ -22,6 +22,7 @@
 #include "mesh.hpp"
 #include "monitor.hpp"
 #include "parameter.hpp"
+#include "periodic.hpp"
 
 namespace {
 
@@ -180,6 +181,8 @@ struct Block {
   corefl::MixArrays mix{}; // species arrays (ns = 0: single-species air)
   double *hstep = nullptr; // per-cell chemistry step size carried between sub-steps
   std::vector<corefl::DevFace> faces; // in boundary-file order
+  corefl::PeriodicPlan periodic{};          // the periodic faces in one launch, where they allow it
+  std::vector<corefl::FaceBatch> outflow;   // the outflow faces, by launch
   std::vector<corefl::DevInner> inner; // block-to-block faces, in inner-file order
   std::vector<int> inner_target;       // their partner blocks
   long part_offset = 0;
@@ -285,15 +288,27 @@ struct corefl_ctx {
 
   void apply_bcs(Block &b, hipStream_t s) {
     // DBoundCond::apply_boundary_conditions order (BoundCond.cu:3489-3619): outflow, inflow, symmetry, periodic.
-    for (int type : {6, 5, 3, 8})
+    for (const auto &f : b.outflow) {
+      if (ns) HIPCHK(corefl::launch_mix_outflow(b.dev, b.mix, f, s));
+      else HIPCHK(corefl::launch_outflow(b.dev, f, s));
+    }
+    for (int type : {5, 3})
       for (size_t q = 0; q < b.faces.size(); ++q) {
         const auto &f = b.faces[q];
         if (f.type != type) continue;
         if (type == 5) HIPCHK(corefl::launch_inflow(b.dev, b.mix, b.inflow[q], s));
-        else if (type == 3) HIPCHK(corefl::launch_symmetry(b.dev, b.mix, f, s));
-        else if (ns) HIPCHK(corefl::launch_mix_boundary(b.dev, b.mix, f, s));
-        else HIPCHK(corefl::launch_boundary(b.dev, f, s));
+        else HIPCHK(corefl::launch_symmetry(b.dev, b.mix, f, s));
       }
+    if (b.periodic.valid) {
+      if (ns) HIPCHK(corefl::launch_mix_periodic(b.dev, b.mix, b.periodic, s));
+      else HIPCHK(corefl::launch_periodic(b.dev, b.periodic, s));
+      return;
+    }
+    for (const auto &f : b.faces) {
+      if (f.type != 8) continue;
+      if (ns) HIPCHK(corefl::launch_mix_periodic_face(b.dev, b.mix, f, s));
+      else HIPCHK(corefl::launch_periodic_face(b.dev, f, s));
+    }
   }
 
   // data_communication (DataCommunication.cu:6-34): every block-to-block face in block and file order, one
@@ -324,9 +339,14 @@ struct corefl_ctx {
     for (auto &b : blocks)
       for (size_t l = 0; l < b.inner.size(); ++l)
         HIPCHK(corefl::launch_inner_viscous_exchange(b.dev, blocks[b.inner_target[l]].dev, b.inner[l], s, nv));
-    for (auto &b : blocks)
+    for (auto &b : blocks) {
+      if (b.periodic.valid) {
+        HIPCHK(corefl::launch_viscous_periodic(b.dev, b.periodic, s, nv));
+        continue;
+      }
       for (const auto &f : b.faces)
         if (f.type == 8) HIPCHK(corefl::launch_viscous_exchange(b.dev, f, s, nv));
+    }
   }
 
   // Chemistry over scale * (*dtp) (a device scalar) in every interior cell of every block (constant density
@@ -998,6 +1018,8 @@ void build(corefl_ctx *ctx, std::vector<corefl::HostBlock> blocks) {
       B.faces.push_back(df);
       B.inflow.push_back(f.type == 5 ? make_inflow(ctx, P, h, f, mech) : corefl::DevInflow{});
     }
+    B.periodic = corefl::periodic_plan(d, B.faces);
+    B.outflow = corefl::face_batches(d, B.faces, 6);
     if (P.get_bool("sponge_layer")) setup_sponge(ctx, P, B, mech);
     for (const auto &f : h.inner) {
       corefl::DevInner di{};

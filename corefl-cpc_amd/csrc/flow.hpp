@@ -28,6 +28,9 @@ struct DevFace {
   int type, face, direction;
 };
 
+struct PeriodicPlan; // the block's periodic sides in one launch (periodic.hpp)
+struct FaceBatch;    // faces filled by one launch (periodic.hpp)
+
 // A block-to-block face on the device (see InnerFace in mesh.hpp).
 struct DevInner {
   int start[3], loop_dir[3], n_point[3];
@@ -70,10 +73,15 @@ struct Scheme {
 
 // Enqueue on `s`.  Each returns hipSuccess or the launch error.
 hipError_t launch_cv_from_bv_all(const DevBlock &b, hipStream_t s);
-hipError_t launch_boundary(const DevBlock &b, const DevFace &f, hipStream_t s);
+// Outflow faces of a block in one launch, its periodic sides in one launch, and one periodic face alone (for blocks
+// without a valid plan).
+hipError_t launch_outflow(const DevBlock &b, const FaceBatch &f, hipStream_t s);
+hipError_t launch_periodic(const DevBlock &b, const PeriodicPlan &p, hipStream_t s);
+hipError_t launch_periodic_face(const DevBlock &b, const DevFace &f, hipStream_t s);
 hipError_t launch_viscous_flux(const DevBlock &b, const Scheme &sc, hipStream_t s);
 // Ghost layers of the collocated viscous fluxes across a periodic face, components 1 .. nv-1.
 hipError_t launch_viscous_exchange(const DevBlock &b, const DevFace &f, hipStream_t s, int nv = 5);
+hipError_t launch_viscous_periodic(const DevBlock &b, const PeriodicPlan &p, hipStream_t s, int nv = 5);
 // inner_communication<Air> / inner_exchange task 1 (DataCommunication.cu:36-103, 458-495) for one face of b
 // whose partner block is t.
 hipError_t launch_inner_exchange(const DevBlock &b, const DevBlock &t, const DevInner &f, hipStream_t s);

@@ -9,6 +9,7 @@
 
 #include <cmath>
 
+#include "periodic.hpp"
 #include "stencil.hpp"
 #include "weno.hpp"
 
@@ -841,6 +842,20 @@ __global__ __launch_bounds__(256) void k_viscous_exchange(DevBlock b, DevFace f,
     for (int a = 0; a < 3; ++a) A[a][ig + l * sz] = A[a][is + l * sz];
 }
 
+// The same exchange over every periodic side at once (periodic.hpp), one thread per orbit and array component.
+struct ScalarOrbit {
+  double *f;
+  __device__ __forceinline__ void load(long node, double (&v)[1]) const { v[0] = f[node]; }
+  __device__ __forceinline__ void store(long node, const double (&v)[1]) const { f[node] = v[0]; }
+};
+
+__global__ __launch_bounds__(256) void k_viscous_periodic(DevBlock b, PeriodicPlan p) {
+  int c[3];
+  if (!periodic_item(p, b.g, blockIdx.x * 256u + threadIdx.x, c)) return;
+  const int a = blockIdx.y % 3, l = 1 + blockIdx.y / 3;
+  periodic_orbit<1>(b, p, c, ScalarOrbit{(a == 0 ? b.fv : (a == 1 ? b.gv : b.hv)) + l * b.sz});
+}
+
 // compute_entropy_fix_delta<Air> (InviscidScheme.cu:269-304) on the interior plus one layer.
 __global__ __launch_bounds__(256) void k_entropy_fix(DevBlock b, Scheme sc) {
   const int i = blockIdx.x * 64 + threadIdx.x - 1, j = blockIdx.y * 4 + threadIdx.y - 1;
@@ -861,14 +876,23 @@ __global__ __launch_bounds__(256) void k_entropy_fix(DevBlock b, Scheme sc) {
 }
 
 // ---------------------------------------------------------------- residual + RK stage
-__device__ __forceinline__ void cons_from_prim(const DevBlock &b, long id) {
+// cv from the primitive state v = rho, u, v, w, p; the fused multiply-adds are written out, so that every kernel
+// that fills a ghost rounds it alike.
+__device__ __forceinline__ void store_cons(const DevBlock &b, long id, const double *v) {
   const long sz = b.sz;
-  const double rho = b.bv[id], u = b.bv[id + sz], v = b.bv[id + 2 * sz], w = b.bv[id + 3 * sz];
-  b.cv[id] = rho;
-  b.cv[id + sz] = rho * u;
-  b.cv[id + 2 * sz] = rho * v;
-  b.cv[id + 3 * sz] = rho * w;
-  b.cv[id + 4 * sz] = 0.5 * (u * u + v * v + w * w) * rho + b.bv[id + 4 * sz] / (kGamma - 1);
+  b.cv[id] = v[0];
+  b.cv[id + sz] = v[0] * v[1];
+  b.cv[id + 2 * sz] = v[0] * v[2];
+  b.cv[id + 3 * sz] = v[0] * v[3];
+  const double uu = fma(v[1], v[1], fma(v[2], v[2], v[3] * v[3]));
+  b.cv[id + 4 * sz] = fma(0.5 * uu, v[0], v[4] / (kGamma - 1));
+}
+
+__device__ __forceinline__ void cons_from_prim(const DevBlock &b, long id) {
+  double v[5];
+#pragma unroll
+  for (int l = 0; l < 5; ++l) v[l] = b.bv[id + l * b.sz];
+  store_cons(b, id, v);
 }
 
 __constant__ double kRkA[3] = {1.0, 0.75, 1.0 / 3.0}; // SSPRK3 (RK.cuh:11-15)
@@ -995,34 +1019,58 @@ __global__ __launch_bounds__(256) void k_update(DevBlock b, int rk, const double
 }
 
 // ---------------------------------------------------------------- boundary conditions
-// apply_outflow without back pressure (BoundCond.cu:2065-2188) and apply_periodic (BoundCond.cu:3033-3083).
-__global__ __launch_bounds__(256) void k_boundary(DevBlock b, DevFace f) {
+struct AirOrbit {
+  const DevBlock &b;
+  __device__ __forceinline__ void load(long node, double (&v)[6]) const {
+#pragma unroll
+    for (int l = 0; l < 6; ++l) v[l] = b.bv[node + l * b.sz];
+  }
+  __device__ __forceinline__ void store(long node, const double (&v)[6]) const {
+#pragma unroll
+    for (int l = 0; l < 6; ++l) b.bv[node + l * b.sz] = v[l];
+    store_cons(b, node, v);
+  }
+};
+
+// apply_periodic (BoundCond.cu:3033-3083) over every periodic side at once (periodic.hpp).
+__global__ __launch_bounds__(256) void k_periodic(DevBlock b, PeriodicPlan p) {
+  int c[3];
+  if (!periodic_item(p, b.g, blockIdx.x * 256u + threadIdx.x, c)) return;
+  periodic_orbit<6>(b, p, c, AirOrbit{b});
+}
+
+// apply_outflow without back pressure (BoundCond.cu:2065-2188) on every outflow face at once: a face's ghosts take the
+// face node's state, which no other item writes.
+__global__ __launch_bounds__(256) void k_outflow(DevBlock b, FaceBatch B) {
+  long node, ghost;
+  if (!face_batch_item(b, B, node, ghost)) return;
+  const AirOrbit op{b};
+  double v[6];
+  op.load(node, v);
+  op.store(ghost, v);
+}
+
+// apply_periodic (BoundCond.cu:3033-3083) of one face, for blocks whose periodic faces are partial or unpaired.
+__global__ __launch_bounds__(256) void k_periodic_face(DevBlock b, DevFace f) {
   FaceItem it;
   if (!face_item(b, f, it)) return;
-  int dv[3] = {0, 0, 0};
+  int dv[3] = {0, 0, 0}, o[3] = {it.i, it.j, it.k};
+  const int ext[3] = {b.mx, b.my, b.mz};
   dv[f.face] = f.direction;
-  const long id = nid(b, it.i, it.j, it.k), sz = b.sz;
+  o[f.face] = f.direction < 0 ? ext[f.face] - 1 : 0;
+  const AirOrbit op{b};
   const int g = it.g;
-  const long ig = nid(b, it.i + g * dv[0], it.j + g * dv[1], it.k + g * dv[2]);
-  if (f.type == 8) {
-    int o[3] = {it.i, it.j, it.k};
-    const int ext[3] = {b.mx, b.my, b.mz};
-    o[f.face] = f.direction < 0 ? ext[f.face] - 1 : 0;
-    if (g == 1) {
-      const long io = nid(b, o[0], o[1], o[2]);
-      for (int l = 0; l < 6; ++l) {
-        const double a = 0.5 * (b.bv[id + l * sz] + b.bv[io + l * sz]);
-        b.bv[id + l * sz] = a;
-        b.bv[io + l * sz] = a;
-      }
-      cons_from_prim(b, id);
-    }
-    const long is = nid(b, o[0] + g * dv[0], o[1] + g * dv[1], o[2] + g * dv[2]);
-    for (int l = 0; l < 6; ++l) b.bv[ig + l * sz] = b.bv[is + l * sz];
-  } else { // zero-gradient outflow
-    for (int l = 0; l < 6; ++l) b.bv[ig + l * sz] = b.bv[id + l * sz];
+  double v[6];
+  if (g == 1) {
+    const long id = nid(b, it.i, it.j, it.k), io = nid(b, o[0], o[1], o[2]);
+    double w[6];
+    op.load(id, v);
+    op.load(io, w);
+    for (int l = 0; l < 6; ++l) b.bv[io + l * b.sz] = v[l] = 0.5 * (v[l] + w[l]);
+    op.store(id, v);
   }
-  cons_from_prim(b, ig);
+  op.load(nid(b, o[0] + g * dv[0], o[1] + g * dv[1], o[2] + g * dv[2]), v);
+  op.store(nid(b, it.i + g * dv[0], it.j + g * dv[1], it.k + g * dv[2]), v);
 }
 
 // One node of a block-to-block face: its index in b and its partner's index in the target block.
@@ -1242,8 +1290,18 @@ static unsigned face_blocks(const DevBlock &b, const DevFace &f) {
   return (unsigned)((n + 255) / 256);
 }
 
-hipError_t launch_boundary(const DevBlock &b, const DevFace &f, hipStream_t s) {
-  k_boundary<<<face_blocks(b, f), 256, 0, s>>>(b, f);
+hipError_t launch_outflow(const DevBlock &b, const FaceBatch &f, hipStream_t s) {
+  k_outflow<<<(f.first[f.n] + 255) / 256, 256, 0, s>>>(b, f);
+  return hipGetLastError();
+}
+
+hipError_t launch_periodic(const DevBlock &b, const PeriodicPlan &p, hipStream_t s) {
+  k_periodic<<<(p.total + 255) / 256, 256, 0, s>>>(b, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_periodic_face(const DevBlock &b, const DevFace &f, hipStream_t s) {
+  k_periodic_face<<<face_blocks(b, f), 256, 0, s>>>(b, f);
   return hipGetLastError();
 }
 
@@ -1270,6 +1328,11 @@ hipError_t launch_viscous_flux(const DevBlock &b, const Scheme &sc, hipStream_t 
 
 hipError_t launch_viscous_exchange(const DevBlock &b, const DevFace &f, hipStream_t s, int nv) {
   k_viscous_exchange<<<face_blocks(b, f), 256, 0, s>>>(b, f, nv);
+  return hipGetLastError();
+}
+
+hipError_t launch_viscous_periodic(const DevBlock &b, const PeriodicPlan &p, hipStream_t s, int nv) {
+  k_viscous_periodic<<<dim3((p.total + 255) / 256, 3 * (nv - 1)), 256, 0, s>>>(b, p);
   return hipGetLastError();
 }
 

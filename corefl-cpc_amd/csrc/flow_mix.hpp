@@ -28,7 +28,10 @@ struct MixArrays {
 };
 
 hipError_t launch_mix_cv_from_bv_all(const DevBlock &b, const MixArrays &x, hipStream_t s);
-hipError_t launch_mix_boundary(const DevBlock &b, const MixArrays &x, const DevFace &f, hipStream_t s);
+// Outflow faces of a block, its periodic sides, and one periodic face alone, as the single-species launchers.
+hipError_t launch_mix_outflow(const DevBlock &b, const MixArrays &x, const FaceBatch &f, hipStream_t s);
+hipError_t launch_mix_periodic(const DevBlock &b, const MixArrays &x, const PeriodicPlan &p, hipStream_t s);
+hipError_t launch_mix_periodic_face(const DevBlock &b, const MixArrays &x, const DevFace &f, hipStream_t s);
 // inner_communication<Mixture> (DataCommunication.cu:36-103) for one face of b whose partner block is t.
 hipError_t launch_mix_inner_exchange(const DevBlock &b, const MixArrays &x, const DevBlock &t, const MixArrays &y,
                                      const DevInner &f, hipStream_t s);

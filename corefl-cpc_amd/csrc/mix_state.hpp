@@ -17,29 +17,36 @@ namespace mixdev {
 
 constexpr int NS = 9;
 
-__device__ inline void mix_cons(const DevBlock &b, const MixArrays &x, long id) {
+// cv and the acoustic speed of node id from its primitive state v = rho, u, v, w, p, T and mass fractions y.
+__device__ inline void store_cons(const DevBlock &b, const MixArrays &x, long id, const double *v, const double *y) {
   const long sz = b.sz;
   const ChemMech &m = *x.mech;
-  const double rho = b.bv[id], u = b.bv[id + sz], v = b.bv[id + 2 * sz], w = b.bv[id + 3 * sz];
-  const double p = b.bv[id + 4 * sz], T = b.bv[id + 5 * sz];
   double h[NS], cp[NS];
-  chemdev::h_cp<NS>(m, T, h, cp);
-  double E = 0.5 * (u * u + v * v + w * w), imw = 0, cpt = 0;
+  chemdev::h_cp<NS>(m, v[5], h, cp);
+  double E = 0.5 * (v[1] * v[1] + v[2] * v[2] + v[3] * v[3]), imw = 0, cpt = 0;
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
-    const double y = x.sv[id + l * sz];
-    E += h[l] * y;
-    imw += y * m.imw[l];
-    cpt += y * cp[l];
-    b.cv[id + (5 + l) * sz] = rho * y;
+    E += h[l] * y[l];
+    imw += y[l] * m.imw[l];
+    cpt += y[l] * cp[l];
+    b.cv[id + (5 + l) * sz] = v[0] * y[l];
   }
-  b.cv[id] = rho;
-  b.cv[id + sz] = rho * u;
-  b.cv[id + 2 * sz] = rho * v;
-  b.cv[id + 3 * sz] = rho * w;
-  b.cv[id + 4 * sz] = E * rho - p;
+  b.cv[id] = v[0];
+  b.cv[id + sz] = v[0] * v[1];
+  b.cv[id + 2 * sz] = v[0] * v[2];
+  b.cv[id + 3 * sz] = v[0] * v[3];
+  b.cv[id + 4 * sz] = E * v[0] - v[4];
   const double R = chemdev::kRu * imw;
-  x.snd[id] = sqrt(cpt / (cpt - R) * R * T);
+  x.snd[id] = sqrt(cpt / (cpt - R) * R * v[5]);
+}
+
+__device__ inline void mix_cons(const DevBlock &b, const MixArrays &x, long id) {
+  double v[6], y[NS];
+#pragma unroll
+  for (int l = 0; l < 6; ++l) v[l] = b.bv[id + l * b.sz];
+#pragma unroll
+  for (int l = 0; l < NS; ++l) y[l] = x.sv[id + l * b.sz];
+  store_cons(b, x, id, v, y);
 }
 
 } // namespace mixdev
