@@ -393,13 +393,18 @@ struct corefl_ctx {
     if (!rhs_only) communicate(s);
   }
 
-  // Slab thickness (planes) of the air stages in z-slabs (setup key stage_slab_planes; -1: two march lengths);
-  // 0 when that is 0 or a block is two-dimensional or too thin.
+  // Slab thickness (planes) of the air stages in z-slabs (setup key stage_slab_planes).  -1: two march lengths where a
+  // slab still gives each direction's flux launch 2048 work-groups, four rounds of the 512 the chip holds, and
+  // unsliced stages below that: the slabs' updates then leave most CUs idle (Taylor-Green steps on n^3 nodes, sliced
+  // against unsliced: 33^3 415 and 340 us, 129^3 2780 and 2625, 161^3 5096 and 5016, 193^3 8104 and 8335, 257^3 18.6
+  // and 19.6 ms).  0 when that is 0 or a block is two-dimensional or too thin.
   int slab_planes() const {
     const int P = slab_setting < 0 ? 2 * corefl::march_planes() : slab_setting;
     if (P == 0) return 0;
-    for (const auto &b : blocks)
+    for (const auto &b : blocks) {
       if (b.dev.dim != 3 || b.dev.mz < 2 * P || (b.dev.mz + P - 1) / P > kMaxSlabs) return 0;
+      if (slab_setting < 0 && (long)(b.dev.mx * b.dev.my + 255) / 256 * P < 2048) return 0;
+    }
     return P;
   }
 
@@ -422,7 +427,7 @@ struct corefl_ctx {
       const int n_slab = (b.dev.mz + P - 1) / P;
       if (scheme.inviscid_scheme == 2) HIPCHK(corefl::launch_entropy_fix(b.dev, scheme, side));
       for (int q = 0; q < n_slab; ++q) {
-        for (int d = 0; d < 3; ++d) HIPCHK(corefl::launch_inviscid_flux(b.dev, scheme, d, side, q * P, (q + 1) * P));
+        HIPCHK(corefl::launch_inviscid_flux(b.dev, scheme, 7u, side, q * P, (q + 1) * P));
         HIPCHK(hipEventRecord(ev_slab[q], side));
       }
       for (int q = 0; q < n_slab; ++q) {
@@ -467,7 +472,7 @@ struct corefl_ctx {
         for (int d = 0; d < b.dev.dim; ++d) HIPCHK(corefl::launch_mix_inviscid_flux(b.dev, b.mix, scheme, d, s));
       } else {
         if (scheme.inviscid_scheme == 2) HIPCHK(corefl::launch_entropy_fix(b.dev, scheme, s));
-        for (int d = 0; d < b.dev.dim; ++d) HIPCHK(corefl::launch_inviscid_flux(b.dev, scheme, d, s));
+        HIPCHK(corefl::launch_inviscid_flux(b.dev, scheme, 7u, s));
       }
     }
     if (visc) HIPCHK(hipStreamWaitEvent(s, ev_join, 0));
@@ -1715,9 +1720,9 @@ int corefl_profile_kernels(corefl_ctx *ctx, int reps, double *ms_out, int n_out)
         timed(1, [&] { ctx->viscous_exchange(s); });
       }
       if (sc.inviscid_scheme == 2) HIPCHK(corefl::launch_entropy_fix(b.dev, sc, s));
-      timed(2, [&] { HIPCHK(corefl::launch_inviscid_flux(b.dev, sc, 0, s)); });
-      timed(3, [&] { HIPCHK(corefl::launch_inviscid_flux(b.dev, sc, 1, s)); });
-      if (b.dev.dim == 3) timed(4, [&] { HIPCHK(corefl::launch_inviscid_flux(b.dev, sc, 2, s)); });
+      timed(2, [&] { HIPCHK(corefl::launch_inviscid_flux(b.dev, sc, 1u, s)); });
+      timed(3, [&] { HIPCHK(corefl::launch_inviscid_flux(b.dev, sc, 2u, s)); });
+      if (b.dev.dim == 3) timed(4, [&] { HIPCHK(corefl::launch_inviscid_flux(b.dev, sc, 4u, s)); });
       timed(5, [&] { HIPCHK(corefl::launch_update(b.dev, sc, 1, ctx->dt_dev, false, s)); });
       timed(6, [&] { ctx->apply_bcs(b, s); });
       timed(7, [&] { ctx->enqueue_dt(s, 0); });

@@ -8,12 +8,25 @@
 #include "flow.hpp"
 
 #include <cmath>
+#include <type_traits>
 
 #include "periodic.hpp"
 #include "stencil.hpp"
 #include "weno.hpp"
 
 namespace corefl {
+
+// COREFL_KZ, or 0.
+static int march_env() {
+  static const int kz = [] {
+    const char *e = std::getenv("COREFL_KZ");
+    const int v = e ? std::atoi(e) : 0;
+    return !e ? 0 : v < 1 ? 1 : v > 256 ? 256 : v;
+  }();
+  return kz;
+}
+static bool march_fixed() { return march_env() > 0; }
+int march_planes() { return march_fixed() ? march_env() : 8; }
 
 namespace {
 
@@ -55,10 +68,10 @@ inline TileGrid plane_grid(int nx, int ny, int gz, int fast, int z0) {
   return TileGrid{(nx * ny + 255) / 256, 1, gz, fast, z0, nx, ny};
 }
 
-__device__ __forceinline__ bool xcd_tile(const TileGrid &t, Tile &out) {
+__device__ __forceinline__ bool xcd_tile(const TileGrid &t, unsigned block, Tile &out) {
   const unsigned total = (unsigned)t.gx * t.gz;
   const unsigned per = (total + 7) / 8;
-  const unsigned n = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  const unsigned n = (block % 8) * per + block / 8;
   if (n >= total) return false;
   unsigned x;
   if (t.fast == 2) {
@@ -78,6 +91,35 @@ __device__ __forceinline__ bool xcd_tile(const TileGrid &t, Tile &out) {
 inline unsigned tile_blocks(const TileGrid &t) {
   const unsigned total = (unsigned)t.gx * t.gz;
   return 8 * ((total + 7) / 8);
+}
+
+// The three directions of an interface kernel in one launch: work-groups [0, end[0]) take the x interfaces,
+// [end[0], end[1]) the y and [end[1], end[2]) the z ones.  Each count is a multiple of 8, so a direction's tiles keep
+// their XCDs.  Direction by direction a small block leaves most of the chip idle three times over (129 work-groups for
+// each direction of a 33^3 block) and a large one pays three partly filled last rounds.  One launch takes 13 us on 33^3
+// nodes (7.5 us a direction before) and 601 us on 129^3 (3 x 237).
+struct SweepGrid {
+  TileGrid t[3];
+  unsigned end[3];
+};
+
+inline unsigned sweep_blocks(SweepGrid &g) {
+  unsigned n = 0;
+  for (int d = 0; d < 3; ++d) g.end[d] = n += g.t[d].gz > 0 ? tile_blocks(g.t[d]) : 0;
+  return n;
+}
+
+// Calls f(direction, tile grid, work-group within it) with the direction as a compile-time constant.
+template<class F> __device__ __forceinline__ void sweep(const SweepGrid &g, F &&f) {
+  const unsigned n = blockIdx.x;
+  if (n < g.end[0]) f(std::integral_constant<int, 0>{}, g.t[0], n);
+  else if (n < g.end[1]) f(std::integral_constant<int, 1>{}, g.t[1], n - g.end[0]);
+  else f(std::integral_constant<int, 2>{}, g.t[2], n - g.end[1]);
+}
+
+// Interface fluxes along DIR go to this array.
+template<int DIR> __device__ __forceinline__ double *flux_array(const DevBlock &b) {
+  return DIR == 0 ? b.fx : (DIR == 1 ? b.fy : b.fz);
 }
 
 // ---------------------------------------------------------------- Riemann solvers
@@ -266,9 +308,10 @@ __device__ __forceinline__ void to_primitive(const double *q, double *p) {
 // t and t+1 (rows as in WENO.cu:73-124), reconstruction is one-sided WENO in those fields,
 // back-projection is the explicit R of WENO.cu:229-243, then the chosen Riemann solver.
 template<int DIR, int R, int RS>
-__global__ __launch_bounds__(256) void k_inviscid(DevBlock b, Scheme sc, double *F, TileGrid tg) {
+__device__ __forceinline__ void inviscid_flux(const DevBlock &b, const Scheme &sc, const TileGrid &tg, unsigned block) {
+  double *F = flux_array<DIR>(b);
   Tile t;
-  if (!xcd_tile(tg, t)) return;
+  if (!xcd_tile(tg, block, t)) return;
   int i = t.i, j = t.j, k = t.z;
   if constexpr (DIR == 0) i -= 1;
   else if constexpr (DIR == 1) j -= 1;
@@ -387,6 +430,11 @@ __global__ __launch_bounds__(256) void k_inviscid(DevBlock b, Scheme sc, double 
   for (int l = 0; l < 5; ++l) F[id + l * sz] = fc[l];
 }
 
+template<int R, int RS>
+__global__ __launch_bounds__(256) void k_inviscid(DevBlock b, Scheme sc, SweepGrid g) {
+  sweep(g, [&](auto dir, const TileGrid &t, unsigned n) { inviscid_flux<dir.value, R, RS>(b, sc, t, n); });
+}
+
 // ---------------------------------------------------------------- primitive reconstruction (air)
 // minmod limiter (Limiter.cuh:8-41; limiter 0 and 1 are both minmod).
 __device__ __forceinline__ double minmod(double a, double c) {
@@ -399,9 +447,10 @@ __device__ __forceinline__ double minmod(double a, double c) {
 // (Reconstruction.cu:5-44: REC 1 first order, 2 MUSCL with kappa = 1/3, 3 NND2, both with minmod), the total
 // energy of each side from its reconstructed state (InviscidScheme.cu:212-217), then the Riemann solver RS.
 template<int DIR, int REC, int RS>
-__global__ __launch_bounds__(256) void k_inviscid_pv(DevBlock b, Scheme sc, double *F, TileGrid tg) {
+__device__ __forceinline__ void inviscid_pv_flux(const DevBlock &b, const Scheme &sc, const TileGrid &tg, unsigned block) {
+  double *F = flux_array<DIR>(b);
   Tile t;
-  if (!xcd_tile(tg, t)) return;
+  if (!xcd_tile(tg, block, t)) return;
   int i = t.i, j = t.j, k = t.z;
   if constexpr (DIR == 0) i -= 1;
   else if constexpr (DIR == 1) j -= 1;
@@ -448,6 +497,11 @@ __global__ __launch_bounds__(256) void k_inviscid_pv(DevBlock b, Scheme sc, doub
   for (int l = 0; l < 5; ++l) F[id + l * sz] = fc[l];
 }
 
+template<int REC, int RS>
+__global__ __launch_bounds__(256) void k_inviscid_pv(DevBlock b, Scheme sc, SweepGrid g) {
+  sweep(g, [&](auto dir, const TileGrid &t, unsigned n) { inviscid_pv_flux<dir.value, REC, RS>(b, sc, t, n); });
+}
+
 // ---------------------------------------------------------------- LLF flux-splitting WENO (air)
 // inviscid_scheme 51/71: component-wise WENO5/WENO7 of the locally split fluxes (WENO.cu:890-990);
 // 52/72: characteristic WENO of the fluxes split with the largest spectral radius on the stencil
@@ -456,9 +510,10 @@ __global__ __launch_bounds__(256) void k_inviscid_pv(DevBlock b, Scheme sc, doub
 // t-ngg+1 .. t+ngg all have a shock sensor at or below the threshold take the linear upwind weights (UD5/UD7);
 // the others, and all of them when it is off, the nonlinear ones.  F receives the interface flux at node t.
 template<int DIR, int R, bool CH>
-__global__ __launch_bounds__(256, 2) void k_fsweno(DevBlock b, Scheme sc, double *F, TileGrid tg) {
+__device__ __forceinline__ void fsweno_flux(const DevBlock &b, const Scheme &sc, const TileGrid &tg, unsigned block) {
+  double *F = flux_array<DIR>(b);
   Tile t;
-  if (!xcd_tile(tg, t)) return;
+  if (!xcd_tile(tg, block, t)) return;
   int i = t.i, j = t.j, k = t.z;
   if constexpr (DIR == 0) i -= 1;
   else if constexpr (DIR == 1) j -= 1;
@@ -634,6 +689,11 @@ __global__ __launch_bounds__(256, 2) void k_fsweno(DevBlock b, Scheme sc, double
   }
 }
 
+template<int R, bool CH>
+__global__ __launch_bounds__(256, 2) void k_fsweno(DevBlock b, Scheme sc, SweepGrid g) {
+  sweep(g, [&](auto dir, const TileGrid &t, unsigned n) { fsweno_flux<dir.value, R, CH>(b, sc, t, n); });
+}
+
 // ---------------------------------------------------------------- viscous terms
 using stencil::dd;
 using stencil::dd_closure;
@@ -655,9 +715,9 @@ __device__ __forceinline__ double sutherland(double T) {
 // the two nodes' averages; the derivative along DIR is the nodes' difference, the transverse ones the
 // average of the two nodes' central differences (none along z on 2D blocks); viscosity the nodes' average.
 template<int DIR>
-__global__ __launch_bounds__(256) void k_viscous_face(DevBlock b, Scheme sc, TileGrid tg) {
+__device__ __forceinline__ void viscous_face(const DevBlock &b, const Scheme &sc, const TileGrid &tg, unsigned block) {
   Tile t;
-  if (!xcd_tile(tg, t)) return;
+  if (!xcd_tile(tg, block, t)) return;
   int i = t.i, j = t.j, k = t.z;
   if constexpr (DIR == 0) i -= 1;
   else if constexpr (DIR == 1) j -= 1;
@@ -711,11 +771,15 @@ __global__ __launch_bounds__(256) void k_viscous_face(DevBlock b, Scheme sc, Til
   F[id + 4 * sz] = um * f1 + vm * f2 + wm * f3 + kc * (kj[0] * d[3][0] + kj[1] * d[3][1] + kj[2] * d[3][2]);
 }
 
+__global__ __launch_bounds__(256) void k_viscous_face(DevBlock b, Scheme sc, SweepGrid g) {
+  sweep(g, [&](auto dir, const TileGrid &t, unsigned n) { viscous_face<dir.value>(b, sc, t, n); });
+}
+
 // compute_viscous_flux_collocated<Air, ORDER> (ViscousScheme.cu:309-408): node fluxes fv/gv/hv[1..4].
 template<int ORDER>
 __global__ __launch_bounds__(256) void k_viscous_flux(DevBlock b, Scheme sc, TileGrid tg, int kz) {
   Tile t;
-  if (!xcd_tile(tg, t)) return;
+  if (!xcd_tile(tg, blockIdx.x, t)) return;
   const int i = t.i, j = t.j;
   if (i >= b.mx || j >= b.my) return;
   const int k0 = t.z * kz, k1 = min(k0 + kz, b.mz);
@@ -905,7 +969,7 @@ template<int ORDER, bool RHS_ONLY>
 __global__ __launch_bounds__(256) void k_update(DevBlock b, int rk, const double *__restrict__ dtp, TileGrid tg,
                                                 int kz) {
   Tile t;
-  if (!xcd_tile(tg, t)) return;
+  if (!xcd_tile(tg, blockIdx.x, t)) return;
   const int i = t.i, j = t.j;
   if (i >= b.mx || j >= b.my) return;
   const int k0 = t.z * kz, k1 = min(k0 + kz, b.mz);
@@ -1212,13 +1276,13 @@ __global__ void k_time_advance(double *time, const double *dt) { time[0] += dt[0
 // step are indexed by workgroup in this grid
 dim3 node_grid(const DevBlock &b) { return dim3((unsigned)((b.mx * b.my + 255) / 256), 1, b.mz); }
 
-// Planes per column of the z-marching kernels.
-int march_kz() {
-  static const int kz = [] {
-    const char *e = std::getenv("COREFL_KZ");
-    const int v = e ? std::atoi(e) : 8;
-    return v < 1 ? 1 : v > 256 ? 256 : v;
-  }();
+// Planes per column of the z-marching kernels: at most march_planes(), and halved while the launch would have fewer
+// than eight work-groups per CU, since a column's planes follow one another (COREFL_KZ fixes it).  At 33^3 nodes the
+// update takes 10 us in single planes and 100 us in eight, at 257^3 eight are the best (1.62 ms, 1.93 in one).
+int march_kz(const DevBlock &b) {
+  int kz = march_planes();
+  if (!march_fixed())
+    while (kz > 1 && (long)((b.mx * b.my + 255) / 256) * ((b.mz + kz - 1) / kz) < 2048) kz /= 2;
   return kz;
 }
 
@@ -1308,18 +1372,16 @@ hipError_t launch_periodic_face(const DevBlock &b, const DevFace &f, hipStream_t
 hipError_t launch_viscous_flux(const DevBlock &b, const Scheme &sc, hipStream_t s) {
   const dim3 tpb(64, 4, 1);
   if (sc.viscous_order == 2) {
-    // one launch per face direction, over the faces -1/2 .. m-1/2 along it
-    const TileGrid tx = plane_grid(b.mx + 1, b.my, b.mz, 0, 0);
-    const TileGrid ty = plane_grid(b.mx, b.my + 1, b.mz, 0, 0);
-    k_viscous_face<0><<<tile_blocks(tx), tpb, 0, s>>>(b, sc, tx);
-    k_viscous_face<1><<<tile_blocks(ty), tpb, 0, s>>>(b, sc, ty);
-    if (b.dim == 3) {
-      const TileGrid tz = plane_grid(b.mx, b.my, b.mz + 1, 2, 0);
-      k_viscous_face<2><<<tile_blocks(tz), tpb, 0, s>>>(b, sc, tz);
-    }
+    // the faces -1/2 .. m-1/2 along each direction
+    SweepGrid g{};
+    g.t[0] = plane_grid(b.mx + 1, b.my, b.mz, 0, 0);
+    g.t[1] = plane_grid(b.mx, b.my + 1, b.mz, 0, 0);
+    if (b.dim == 3) g.t[2] = plane_grid(b.mx, b.my, b.mz + 1, 2, 0);
+    const unsigned nb = sweep_blocks(g);
+    k_viscous_face<<<nb, tpb, 0, s>>>(b, sc, g);
     return hipGetLastError();
   }
-  const int kz = march_kz();
+  const int kz = march_kz(b);
   const TileGrid tm = march_tiles(b, kz);
   if (sc.viscous_order == 8) k_viscous_flux<8><<<tile_blocks(tm), tpb, 0, s>>>(b, sc, tm, kz);
   else k_viscous_flux<4><<<tile_blocks(tm), tpb, 0, s>>>(b, sc, tm, kz);
@@ -1358,94 +1420,61 @@ hipError_t launch_entropy_fix(const DevBlock &b, const Scheme &sc, hipStream_t s
   return hipGetLastError();
 }
 
-template<int DIR, int R>
-static void dispatch_rs(const DevBlock &b, const Scheme &sc, dim3 grid, double *F, hipStream_t s, int z0) {
+template<int R>
+static void dispatch_rs(const DevBlock &b, const Scheme &sc, const SweepGrid &g, unsigned nb, hipStream_t s) {
   const dim3 tpb(64, 4, 1);
-  const TileGrid tg = plane_grid((int)grid.x, (int)grid.y, (int)grid.z, DIR == 2 ? 2 : 0, z0);
-  const unsigned nb = tile_blocks(tg);
   switch (sc.inviscid_scheme) {
-    case 1: k_inviscid<DIR, R, 1><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    case 2: k_inviscid<DIR, R, 2><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    case 4: k_inviscid<DIR, R, 4><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    default: k_inviscid<DIR, R, 3><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
+    case 1: k_inviscid<R, 1><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    case 2: k_inviscid<R, 2><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    case 4: k_inviscid<R, 4><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    default: k_inviscid<R, 3><<<nb, tpb, 0, s>>>(b, sc, g); break;
   }
 }
 
-template<int DIR, int REC>
-static void dispatch_pv(const DevBlock &b, const Scheme &sc, dim3 grid, double *F, hipStream_t s, int z0) {
+template<int REC>
+static void dispatch_pv(const DevBlock &b, const Scheme &sc, const SweepGrid &g, unsigned nb, hipStream_t s) {
   const dim3 tpb(64, 4, 1);
-  const TileGrid tg = plane_grid((int)grid.x, (int)grid.y, (int)grid.z, DIR == 2 ? 2 : 0, z0);
-  const unsigned nb = tile_blocks(tg);
   switch (sc.inviscid_scheme) {
-    case 1: k_inviscid_pv<DIR, REC, 1><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    case 2: k_inviscid_pv<DIR, REC, 2><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    case 4: k_inviscid_pv<DIR, REC, 4><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    default: k_inviscid_pv<DIR, REC, 3><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
+    case 1: k_inviscid_pv<REC, 1><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    case 2: k_inviscid_pv<REC, 2><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    case 4: k_inviscid_pv<REC, 4><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    default: k_inviscid_pv<REC, 3><<<nb, tpb, 0, s>>>(b, sc, g); break;
   }
 }
 
-template<int DIR>
-static void dispatch_pv_rec(const DevBlock &b, const Scheme &sc, dim3 grid, double *F, hipStream_t s, int z0) {
-  if (sc.reconstruction == 1) dispatch_pv<DIR, 1>(b, sc, grid, F, s, z0);
-  else if (sc.reconstruction == 2) dispatch_pv<DIR, 2>(b, sc, grid, F, s, z0);
-  else dispatch_pv<DIR, 3>(b, sc, grid, F, s, z0);
-}
-
-template<int DIR>
-static void dispatch_fs(const DevBlock &b, const Scheme &sc, dim3 grid, double *F, hipStream_t s, int z0) {
+static void dispatch_fs(const DevBlock &b, const Scheme &sc, const SweepGrid &g, unsigned nb, hipStream_t s) {
   const dim3 tpb(64, 4, 1);
-  const TileGrid tg = plane_grid((int)grid.x, (int)grid.y, (int)grid.z, DIR == 2 ? 2 : 0, z0);
-  const unsigned nb = tile_blocks(tg);
   switch (sc.inviscid_scheme) {
-    case 51: k_fsweno<DIR, 3, false><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    case 52: k_fsweno<DIR, 3, true><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    case 71: k_fsweno<DIR, 4, false><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
-    default: k_fsweno<DIR, 4, true><<<nb, tpb, 0, s>>>(b, sc, F, tg); break;
+    case 51: k_fsweno<3, false><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    case 52: k_fsweno<3, true><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    case 71: k_fsweno<4, false><<<nb, tpb, 0, s>>>(b, sc, g); break;
+    default: k_fsweno<4, true><<<nb, tpb, 0, s>>>(b, sc, g); break;
   }
 }
 
-hipError_t launch_inviscid_flux(const DevBlock &b, const Scheme &sc, int dir, hipStream_t s, int kb, int ke) {
+hipError_t launch_inviscid_flux(const DevBlock &b, const Scheme &sc, unsigned dirs, hipStream_t s, int kb, int ke) {
   // the interfaces of the node planes [kb, ke): F(i+1/2) stored at node i for i = -1 .. mx-1 (x), likewise in y; in
   // z the interfaces k + 1/2 of planes kb .. ke-1, and also -1/2 when kb = 0 (tile z = k + 1)
-  const int me = ke < b.mz ? ke : b.mz;
-  dim3 grid; // nodes along i and j, planes along k
-  double *F;
-  int z0 = kb;
-  if (dir == 0) {
-    grid = dim3(b.mx + 1, b.my, me - kb);
-    F = b.fx;
-  } else if (dir == 1) {
-    grid = dim3(b.mx, b.my + 1, me - kb);
-    F = b.fy;
-  } else {
-    z0 = kb == 0 ? 0 : kb + 1;
-    grid = dim3(b.mx, b.my, me + 1 - z0);
-    F = b.fz;
-  }
-  if ((int)grid.z <= 0) return hipSuccess;
-  if (sc.inviscid_scheme > 50) {
-    if (dir == 0) dispatch_fs<0>(b, sc, grid, F, s, z0);
-    else if (dir == 1) dispatch_fs<1>(b, sc, grid, F, s, z0);
-    else dispatch_fs<2>(b, sc, grid, F, s, z0);
-    return hipGetLastError();
-  }
-  if (sc.reconstruction >= 1 && sc.reconstruction <= 3) {
-    if (dir == 0) dispatch_pv_rec<0>(b, sc, grid, F, s, z0);
-    else if (dir == 1) dispatch_pv_rec<1>(b, sc, grid, F, s, z0);
-    else dispatch_pv_rec<2>(b, sc, grid, F, s, z0);
-    return hipGetLastError();
-  }
-  const bool w7 = sc.reconstruction == 5;
-  if (dir == 0) w7 ? dispatch_rs<0, 4>(b, sc, grid, F, s, z0) : dispatch_rs<0, 3>(b, sc, grid, F, s, z0);
-  else if (dir == 1) w7 ? dispatch_rs<1, 4>(b, sc, grid, F, s, z0) : dispatch_rs<1, 3>(b, sc, grid, F, s, z0);
-  else w7 ? dispatch_rs<2, 4>(b, sc, grid, F, s, z0) : dispatch_rs<2, 3>(b, sc, grid, F, s, z0);
+  const int me = ke < b.mz ? ke : b.mz, z0 = kb == 0 ? 0 : kb + 1;
+  SweepGrid g{};
+  if (dirs & 1u) g.t[0] = plane_grid(b.mx + 1, b.my, me - kb, 0, kb);
+  if (dirs & 2u) g.t[1] = plane_grid(b.mx, b.my + 1, me - kb, 0, kb);
+  if ((dirs & 4u) && b.dim == 3) g.t[2] = plane_grid(b.mx, b.my, me + 1 - z0, 2, z0);
+  const unsigned nb = sweep_blocks(g);
+  if (nb == 0) return hipSuccess;
+  if (sc.inviscid_scheme > 50) dispatch_fs(b, sc, g, nb, s);
+  else if (sc.reconstruction == 1) dispatch_pv<1>(b, sc, g, nb, s);
+  else if (sc.reconstruction == 2) dispatch_pv<2>(b, sc, g, nb, s);
+  else if (sc.reconstruction == 3) dispatch_pv<3>(b, sc, g, nb, s);
+  else if (sc.reconstruction == 5) dispatch_rs<4>(b, sc, g, nb, s);
+  else dispatch_rs<3>(b, sc, g, nb, s);
   return hipGetLastError();
 }
 
 hipError_t launch_update(const DevBlock &b, const Scheme &sc, int rk, const double *dt_dev, bool rhs_only,
                          hipStream_t s, int kb, int ke) {
   const dim3 tpb(64, 4, 1);
-  const int kz = march_kz();
+  const int kz = march_kz(b);
   TileGrid tg = march_tiles(b, kz);
   // the node planes [kb, ke) (kb a multiple of the march length)
   const int me = ke < b.mz ? ke : b.mz;
@@ -1494,7 +1523,5 @@ hipError_t launch_shock_sensor(const DevBlock &b, const Scheme &sc, hipStream_t 
   k_shock_sensor<<<dim3((b.mx + 63) / 64, (b.my + 3) / 4, b.mz), dim3(64, 4, 1), 0, s>>>(b, sc.shock_sensor, sc.sensor_eps);
   return hipGetLastError();
 }
-
-int march_planes() { return march_kz(); }
 
 } // namespace corefl
