@@ -23,6 +23,15 @@ constexpr int kMlpNp[kMlpLayers] = {128, 128, 128, 128, 32}; // N padded to the 
 // Hidden activation: GELU in its tanh form (the network the specification names) or hard swish.
 constexpr int kActGelu = 0, kActHardSwish = 1;
 
+// Flat parameter layout: W_0 (K_0 x N_0, row-major), b_0, W_1, b_1, ..., W_4, b_4.
+constexpr int mlp_offset(int layer, bool bias) {
+  int o = 0;
+  for (int l = 0; l < layer; ++l) o += kMlpK[l] * kMlpN[l] + kMlpN[l];
+  return bias ? o + kMlpK[layer] * kMlpN[layer] : o;
+}
+constexpr int kMlpParams = mlp_offset(4, true) + kMlpOut;
+constexpr int kMlpBackN[kMlpLayers] = {0, 128, 128, 128, 16}; // depth of the layers' backward products
+
 struct MlpDev {
   const unsigned short *wt[kMlpLayers];
   const float *bias[kMlpLayers];
@@ -65,46 +74,51 @@ constexpr int kProjTableEntries = 512, kProjTableStride = 17;
 // E E^T is singular.
 bool projection_tables(const ChemMech &mech, ElementMatrix &em, std::vector<double> &table);
 
-// C = A B with A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn] in BF16; FP32 accumulation.
-enum GemmEpilogue {
-  kEpFwdHidden = 0, // z = acc + bias: C (FP32) = z, Cb (BF16) = act(z)
-  kEpFwdOut = 1,    // C = acc + bias
-  kEpBwdData = 2,   // Cb = acc * act'(zprev)
-  kEpAtomic = 3     // C += acc (split over K by gridDim.z)
+// One training step (or gradient, or forward pass) of a mini-batch.  Rows are handled 32 at a time; the arrays that the
+// weight gradients contract over the batch are stored with eight consecutive rows of a neuron together, as the MFMA
+// takes them (blocks of 32 neurons x 16 rows; ld rows in all, a multiple of 64).
+constexpr int kTrainRows = 32;                       // rows of a work-group of the forward / backward kernel
+// parts of a batch of B rows whose weight gradients are summed apart, at most
+inline int train_max_chunks(int B) { return B <= 16384 ? 16 : 64; }
+// BF16 copies of the weights: W^T [Np][Kp] for inference, and in blocks of one MFMA operand each the rows of W^T for the
+// forward pass of the training and the rows of W (layers 1..4, N padded to 16 in layer 4) for its backward pass.
+struct WeightCopies {
+  unsigned short *wt[kMlpLayers], *wf[kMlpLayers], *wb[kMlpLayers];
 };
 
-struct GemmArgs {
-  int M, N, K;
-  const unsigned short *A;
-  long sam, sak;
-  const unsigned short *B;
-  long sbk, sbn;
-  int ep;
-  float *C;
-  long ldc;
-  unsigned short *Cb;
-  long ldcb;
-  const float *bias;
-  const float *zprev;
-  long ldz;
-  int k_chunk; // K extent of one gridDim.z slice (multiple of 32); K for the non-atomic epilogues
-  int act;     // hidden activation of the forward and data-gradient epilogues
+struct TrainArgs {
+  int B;                                             // rows of the mini-batch
+  const float *X, *Y;                                // data set [n][12], [n][10]; Y null: forward only
+  long n;                                            // rows of the data set
+  unsigned long long seed;                           // row i of the batch is data row i (0), or hash(seed, step, i) mod n
+  long step;
+  const unsigned short *wf[kMlpLayers], *wb[kMlpLayers]; // as in WeightCopies
+  const float *bias[kMlpLayers];
+  unsigned short *HT[kMlpLayers];                    // inputs of layer l, 32 or 128 neurons x ld
+  unsigned short *GT[kMlpLayers];                    // gradients of layer l's pre-activations, 128 or 32 neurons x ld
+  long ld;
+  float *loss_part;                                  // one partial loss per work-group
+  float *out;                                        // forward only: [B][10]
+  int act;
 };
-
-hipError_t launch_gemm(const GemmArgs &a, hipStream_t s);
-// Mini-batch assembly: rows idx_i of X [n][12] -> BF16 H0 [B][16] (zero padded), Y [n][10] -> Yb [B][10];
-// idx_i = i when seed == 0, else a hash of (seed, step, i) modulo n.
-hipError_t launch_gather(const float *X, const float *Y, long n, unsigned long long seed, long step, int B,
-                         unsigned short *H0, float *Yb, hipStream_t s);
-// G = BF16(2 (out - y) / (B * 10)); *loss += mean squared error.
-hipError_t launch_loss(const float *out, const float *Yb, int B, unsigned short *G, float *loss, hipStream_t s);
-// db[n] += sum_b G[b][n] (BF16 G, row stride ldg).
-hipError_t launch_colsum(const unsigned short *G, int B, int N, long ldg, float *db, hipStream_t s);
-// Adam on n FP32 parameters; when wt != nullptr also writes BF16 W^T (K x N weights, row stride Kp).
-hipError_t launch_adam(float *p, float *m, float *v, const float *g, long n, float lr, float b1, float b2, float eps,
-                       float c1, float c2, unsigned short *wt, int K, int N, int Kp, hipStream_t s);
-hipError_t launch_to_bf16t(const float *W, int K, int N, int Kp, unsigned short *wt, hipStream_t s);
-hipError_t launch_fill(float *p, long n, float v, hipStream_t s);
+// The forward pass, and with Y the loss and the backward pass down to every layer's pre-activation gradient.
+hipError_t launch_train_tile(const TrainArgs &a, hipStream_t s);
+// Weight and bias gradients from HT and GT, chunk by chunk of the batch: part[chunk][flat parameter].
+int train_chunks(int B);
+hipError_t launch_train_grad(const TrainArgs &a, float *part, hipStream_t s);
+// Sums the chunks and the partial losses (loss null: not); grads non-null: the gradient goes there and nothing is
+// updated; else Adam on the flat parameters, with the BF16 copies of the weights.
+struct AdamArgs {
+  const float *part, *loss_part;
+  int chunks, loss_parts;
+  float *loss, *grads;
+  float *p, *m, *v;
+  WeightCopies w;
+  float lr, b1, b2, eps, c1, c2;
+};
+hipError_t launch_train_adam(const AdamArgs &a, hipStream_t s);
+// FP32 weights (flat parameters p) -> the BF16 copies.
+hipError_t launch_pack_weights(const float *p, const WeightCopies &w, hipStream_t s);
 
 // Work arrays of a surrogate chemistry step for n cells: BF16 features [n][16], FP32 outputs [n][10] and
 // the input-range flags [n].

@@ -17,37 +17,16 @@
 
 using namespace corefl;
 
-namespace {
-
-// flat parameter layout: W_0 (K_0 x N_0, row-major), b_0, W_1, b_1, ..., W_4, b_4
-struct Offsets {
-  long w[kMlpLayers], b[kMlpLayers], total;
-  Offsets() {
-    long o = 0;
-    for (int l = 0; l < kMlpLayers; ++l) {
-      w[l] = o;
-      o += (long)kMlpK[l] * kMlpN[l];
-      b[l] = o;
-      o += kMlpN[l];
-    }
-    total = o;
-  }
-};
-const Offsets kOff;
-
-} // namespace
-
 struct corefl_surrogate {
   hipStream_t stream = nullptr;
   int cap = 0; // mini-batch capacity
   float *p = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;
-  unsigned short *wt[kMlpLayers] = {};
+  WeightCopies w{};
   long adam_t = 0;
-  // activations of one mini-batch
-  unsigned short *H[kMlpLayers] = {}; // H[0]: [cap][16]; H[l>0]: [cap][128]
-  float *Z[kMlpLayers - 1] = {};      // pre-activations of the hidden layers, [cap][128]
-  float *out = nullptr, *Yb = nullptr;
-  unsigned short *G4 = nullptr, *Ga = nullptr, *Gb = nullptr;
+  // one mini-batch: layer inputs and pre-activation gradients (ld rows); gradients by chunk; partial losses
+  unsigned short *HT[kMlpLayers] = {}, *GT[kMlpLayers] = {};
+  long ld = 0;
+  float *part = nullptr, *loss_part = nullptr;
   float *loss = nullptr; // per-step losses
   long loss_cap = 0;
   // training set
@@ -84,92 +63,53 @@ template<class T> void dalloc(T **p, size_t count) {
 MlpDev net_of(const corefl_surrogate *s) {
   MlpDev n{};
   for (int l = 0; l < kMlpLayers; ++l) {
-    n.wt[l] = s->wt[l];
-    n.bias[l] = s->p + kOff.b[l];
+    n.wt[l] = s->w.wt[l];
+    n.bias[l] = s->p + mlp_offset(l, true);
   }
   n.act = s->act;
   return n;
 }
 
-GemmArgs gemm(int M, int N, int K, const unsigned short *A, long sam, long sak, const unsigned short *B, long sbk,
-              long sbn, int ep) {
-  GemmArgs a{};
-  a.M = M;
-  a.N = N;
-  a.K = K;
-  a.A = A;
-  a.sam = sam;
-  a.sak = sak;
+TrainArgs train_args(const corefl_surrogate *s, int B, const float *X, const float *Y, long n, unsigned long long seed,
+                     long step) {
+  TrainArgs a{};
   a.B = B;
-  a.sbk = sbk;
-  a.sbn = sbn;
-  a.ep = ep;
-  a.k_chunk = ((K + 31) / 32) * 32;
+  a.X = X;
+  a.Y = Y;
+  a.n = n;
+  a.seed = seed;
+  a.step = step;
+  for (int l = 0; l < kMlpLayers; ++l) {
+    a.wf[l] = s->w.wf[l];
+    a.wb[l] = s->w.wb[l];
+    a.bias[l] = s->p + mlp_offset(l, true);
+    a.HT[l] = s->HT[l];
+    a.GT[l] = s->GT[l];
+  }
+  a.ld = s->ld;
+  a.loss_part = s->loss_part;
+  a.act = s->act;
   return a;
 }
 
-// Forward pass of the B rows in H[0]; outputs in s->out.
-void forward(corefl_surrogate *s, int B) {
-  for (int l = 0; l < kMlpLayers; ++l) {
-    const long ld = l == 0 ? 16 : 128;
-    GemmArgs a = gemm(B, kMlpN[l], kMlpKp[l], s->H[l], ld, 1, s->wt[l], 1, kMlpKp[l],
-                      l < kMlpLayers - 1 ? kEpFwdHidden : kEpFwdOut);
-    a.bias = s->p + kOff.b[l];
-    a.act = s->act;
-    if (l < kMlpLayers - 1) {
-      a.C = s->Z[l];
-      a.ldc = 128;
-      a.Cb = s->H[l + 1];
-      a.ldcb = 128;
-    } else {
-      a.C = s->out;
-      a.ldc = kMlpOut;
-    }
-    HIPCHK(launch_gemm(a, s->stream));
-  }
+AdamArgs adam_args(const corefl_surrogate *s, int B, float *loss) {
+  AdamArgs a{};
+  a.part = s->part;
+  a.loss_part = s->loss_part;
+  a.chunks = train_chunks(B);
+  a.loss_parts = (B + kTrainRows - 1) / kTrainRows;
+  a.loss = loss;
+  a.p = s->p;
+  a.m = s->m;
+  a.v = s->v;
+  a.w = s->w;
+  return a;
 }
 
-// Loss and gradients of the B rows (targets in s->Yb) into s->g; loss added to *loss_slot.
-void backward(corefl_surrogate *s, int B, float *loss_slot) {
-  HIPCHK(launch_fill(s->g, kOff.total, 0.0f, s->stream));
-  HIPCHK(launch_loss(s->out, s->Yb, B, s->G4, loss_slot, s->stream));
-  const unsigned short *G = s->G4;
-  long ldg = kMlpOut;
-  for (int l = kMlpLayers - 1; l >= 0; --l) {
-    const long ldh = l == 0 ? 16 : 128;
-    // dW_l = H_l^T G, split over the batch
-    GemmArgs w = gemm(kMlpK[l], kMlpN[l], B, s->H[l], 1, ldh, G, ldg, 1, kEpAtomic);
-    w.C = s->g + kOff.w[l];
-    w.ldc = kMlpN[l];
-    w.k_chunk = 512;
-    HIPCHK(launch_gemm(w, s->stream));
-    HIPCHK(launch_colsum(G, B, kMlpN[l], ldg, s->g + kOff.b[l], s->stream));
-    if (l > 0) {
-      unsigned short *Gn = (G == s->Ga) ? s->Gb : s->Ga;
-      GemmArgs d = gemm(B, kMlpK[l], kMlpN[l], G, ldg, 1, s->wt[l], kMlpKp[l], 1, kEpBwdData);
-      d.zprev = s->Z[l - 1];
-      d.ldz = 128;
-      d.act = s->act;
-      d.Cb = Gn;
-      d.ldcb = 128;
-      HIPCHK(launch_gemm(d, s->stream));
-      G = Gn;
-      ldg = 128;
-    }
-  }
-}
-
-void adam(corefl_surrogate *s, float lr) {
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  ++s->adam_t;
-  const float c1 = 1.0f - std::pow(b1, (float)s->adam_t), c2 = 1.0f - std::pow(b2, (float)s->adam_t);
-  for (int l = 0; l < kMlpLayers; ++l) {
-    const long nw = (long)kMlpK[l] * kMlpN[l];
-    HIPCHK(launch_adam(s->p + kOff.w[l], s->m + kOff.w[l], s->v + kOff.w[l], s->g + kOff.w[l], nw, lr, b1, b2, eps, c1,
-                       c2, s->wt[l], kMlpK[l], kMlpN[l], kMlpKp[l], s->stream));
-    HIPCHK(launch_adam(s->p + kOff.b[l], s->m + kOff.b[l], s->v + kOff.b[l], s->g + kOff.b[l], kMlpN[l], lr, b1, b2,
-                       eps, c1, c2, nullptr, 0, 1, 0, s->stream));
-  }
+// Loss and gradients of the batch into s->part and s->loss_part.
+void gradients(corefl_surrogate *s, const TrainArgs &a) {
+  HIPCHK(launch_train_tile(a, s->stream));
+  HIPCHK(launch_train_grad(a, s->part, s->stream));
 }
 
 void upload_rows(corefl_surrogate *s, long n, const float *X, const float *Y, float **dX, float **dY) {
@@ -286,20 +226,19 @@ void surrogate_substep(corefl_chem *c, corefl_surrogate *s, const ChemBatch &b, 
 } // namespace corefl
 
 corefl_surrogate::~corefl_surrogate() {
-  for (void *q : {(void *)p, (void *)m, (void *)v, (void *)g, (void *)out, (void *)Yb, (void *)G4, (void *)Ga,
-                  (void *)Gb, (void *)loss, (void *)X, (void *)Y})
+  for (void *q : {(void *)p, (void *)m, (void *)v, (void *)g, (void *)part, (void *)loss_part, (void *)loss,
+                  (void *)X, (void *)Y})
     if (q) (void)hipFree(q);
   for (int l = 0; l < kMlpLayers; ++l) {
-    if (wt[l]) (void)hipFree(wt[l]);
-    if (H[l]) (void)hipFree(H[l]);
-    if (l < kMlpLayers - 1 && Z[l]) (void)hipFree(Z[l]);
+    for (unsigned short *q : {w.wt[l], w.wf[l], w.wb[l], HT[l], GT[l]})
+      if (q) (void)hipFree(q);
   }
   if (stream) (void)hipStreamDestroy(stream);
 }
 
 extern "C" {
 
-long long corefl_surrogate_n_params(void) { return kOff.total; }
+long long corefl_surrogate_n_params(void) { return kMlpParams; }
 
 int corefl_surrogate_create(int batch_capacity, corefl_surrogate **out) {
   return guarded([&] {
@@ -312,20 +251,23 @@ int corefl_surrogate_create(int batch_capacity, corefl_surrogate **out) {
     HIPCHK(hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, 0));
     const int B = batch_capacity;
     s->cap = B;
-    for (float **q : {&s->p, &s->m, &s->v, &s->g}) dalloc(q, (size_t)kOff.total);
-    HIPCHK(hipMemsetAsync(s->m, 0, sizeof(float) * kOff.total, s->stream));
-    HIPCHK(hipMemsetAsync(s->v, 0, sizeof(float) * kOff.total, s->stream));
+    for (float **q : {&s->p, &s->m, &s->v, &s->g}) dalloc(q, (size_t)kMlpParams);
+    HIPCHK(hipMemsetAsync(s->m, 0, sizeof(float) * kMlpParams, s->stream));
+    HIPCHK(hipMemsetAsync(s->v, 0, sizeof(float) * kMlpParams, s->stream));
+    s->ld = (B + 63) / 64 * 64;
+    // zeroed arrays: padding rows and columns of the weights, the unused neurons of the narrow layers
+    auto zeroed = [&](unsigned short **q, size_t n) {
+      dalloc(q, n);
+      HIPCHK(hipMemsetAsync(*q, 0, sizeof(unsigned short) * n, s->stream));
+    };
     for (int l = 0; l < kMlpLayers; ++l) {
-      dalloc(&s->wt[l], (size_t)kMlpNp[l] * kMlpKp[l]);
-      HIPCHK(hipMemsetAsync(s->wt[l], 0, sizeof(unsigned short) * kMlpNp[l] * kMlpKp[l], s->stream));
-      dalloc(&s->H[l], (size_t)B * (l == 0 ? 16 : 128));
-      if (l < kMlpLayers - 1) dalloc(&s->Z[l], (size_t)B * 128);
+      for (unsigned short **q : {&s->w.wt[l], &s->w.wf[l]}) zeroed(q, (size_t)kMlpNp[l] * kMlpKp[l]);
+      if (l) zeroed(&s->w.wb[l], (size_t)kMlpHidden * kMlpBackN[l]);
+      zeroed(&s->HT[l], (size_t)(l == 0 ? 32 : kMlpHidden) * s->ld);
+      zeroed(&s->GT[l], (size_t)kMlpNp[l] * s->ld);
     }
-    dalloc(&s->out, (size_t)B * kMlpOut);
-    dalloc(&s->Yb, (size_t)B * kMlpOut);
-    dalloc(&s->G4, (size_t)B * kMlpOut);
-    dalloc(&s->Ga, (size_t)B * 128);
-    dalloc(&s->Gb, (size_t)B * 128);
+    dalloc(&s->part, (size_t)train_max_chunks(B) * kMlpParams);
+    dalloc(&s->loss_part, (size_t)(B + kTrainRows - 1) / kTrainRows);
     HIPCHK(hipStreamSynchronize(s->stream));
     *out = s.release();
   });
@@ -336,13 +278,12 @@ void corefl_surrogate_destroy(corefl_surrogate *s) { delete s; }
 int corefl_surrogate_set_params(corefl_surrogate *s, const float *params, long long n) {
   return guarded([&] {
     if (!s || !params) throw std::runtime_error("corefl_surrogate_set_params: null argument");
-    if (n != kOff.total) throw std::runtime_error("corefl_surrogate_set_params: expected " + std::to_string(kOff.total));
+    if (n != kMlpParams) throw std::runtime_error("corefl_surrogate_set_params: expected " + std::to_string(kMlpParams));
     HIPCHK(hipMemcpyAsync(s->p, params, sizeof(float) * n, hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemsetAsync(s->m, 0, sizeof(float) * n, s->stream));
     HIPCHK(hipMemsetAsync(s->v, 0, sizeof(float) * n, s->stream));
     s->adam_t = 0;
-    for (int l = 0; l < kMlpLayers; ++l)
-      HIPCHK(launch_to_bf16t(s->p + kOff.w[l], kMlpK[l], kMlpN[l], kMlpKp[l], s->wt[l], s->stream));
+    HIPCHK(launch_pack_weights(s->p, s->w, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
     s->have_params = true;
   });
@@ -351,7 +292,7 @@ int corefl_surrogate_set_params(corefl_surrogate *s, const float *params, long l
 int corefl_surrogate_get_params(corefl_surrogate *s, float *params, long long n) {
   return guarded([&] {
     if (!s || !params) throw std::runtime_error("corefl_surrogate_get_params: null argument");
-    if (n != kOff.total) throw std::runtime_error("corefl_surrogate_get_params: expected " + std::to_string(kOff.total));
+    if (n != kMlpParams) throw std::runtime_error("corefl_surrogate_get_params: expected " + std::to_string(kMlpParams));
     need_params(s);
     HIPCHK(hipMemcpyAsync(params, s->p, sizeof(float) * n, hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -432,12 +373,17 @@ int corefl_surrogate_train(corefl_surrogate *s, int batch, int steps, float lr, 
       dalloc(&s->loss, (size_t)steps);
       s->loss_cap = steps;
     }
-    if (steps) HIPCHK(launch_fill(s->loss, steps, 0.0f, s->stream));
     for (int st = 0; st < steps; ++st) {
-      HIPCHK(launch_gather(s->X, s->Y, s->n_data, seed, s->adam_t, batch, s->H[0], s->Yb, s->stream));
-      forward(s, batch);
-      backward(s, batch, s->loss + st);
-      adam(s, lr);
+      gradients(s, train_args(s, batch, s->X, s->Y, s->n_data, seed, s->adam_t));
+      AdamArgs a = adam_args(s, batch, s->loss + st);
+      ++s->adam_t;
+      a.lr = lr;
+      a.b1 = 0.9f;
+      a.b2 = 0.999f;
+      a.eps = 1e-8f;
+      a.c1 = 1.0f - std::pow(a.b1, (float)s->adam_t);
+      a.c2 = 1.0f - std::pow(a.b2, (float)s->adam_t);
+      HIPCHK(launch_train_adam(a, s->stream));
     }
     if (loss_out && steps)
       HIPCHK(hipMemcpyAsync(loss_out, s->loss, sizeof(float) * steps, hipMemcpyDeviceToHost, s->stream));
@@ -455,12 +401,12 @@ int corefl_surrogate_grad(corefl_surrogate *s, long long n, const float *X, cons
     try {
       upload_rows(s, n, X, Y, &dX, &dY);
       dalloc(&dl, 1);
-      HIPCHK(launch_fill(dl, 1, 0.0f, s->stream));
-      HIPCHK(launch_gather(dX, dY, n, 0, 0, (int)n, s->H[0], s->Yb, s->stream));
-      forward(s, (int)n);
-      backward(s, (int)n, dl);
+      gradients(s, train_args(s, (int)n, dX, dY, n, 0, 0));
+      AdamArgs a = adam_args(s, (int)n, dl);
+      a.grads = s->g;
+      HIPCHK(launch_train_adam(a, s->stream));
       HIPCHK(hipMemcpyAsync(loss, dl, sizeof(float), hipMemcpyDeviceToHost, s->stream));
-      HIPCHK(hipMemcpyAsync(grads, s->g, sizeof(float) * kOff.total, hipMemcpyDeviceToHost, s->stream));
+      HIPCHK(hipMemcpyAsync(grads, s->g, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, s->stream));
       HIPCHK(hipStreamSynchronize(s->stream));
     } catch (...) {
       (void)hipStreamSynchronize(s->stream);
@@ -492,9 +438,10 @@ int corefl_surrogate_forward(corefl_surrogate *s, long long n, const float *X, f
         HIPCHK(e2);
         HIPCHK(e3);
       } else {
-        HIPCHK(launch_gather(dX, dY, n, 0, 0, (int)n, s->H[0], s->Yb, s->stream));
-        forward(s, (int)n);
-        HIPCHK(hipMemcpyAsync(out, s->out, sizeof(float) * n * kMlpOut, hipMemcpyDeviceToHost, s->stream));
+        TrainArgs a = train_args(s, (int)n, dX, nullptr, n, 0, 0);
+        a.out = dY;
+        HIPCHK(launch_train_tile(a, s->stream));
+        HIPCHK(hipMemcpyAsync(out, dY, sizeof(float) * n * kMlpOut, hipMemcpyDeviceToHost, s->stream));
       }
       HIPCHK(hipStreamSynchronize(s->stream));
     } catch (...) {

@@ -59,68 +59,7 @@ template<int ACT> __device__ __forceinline__ float act_grad(float z) {
   }
 }
 
-// ------------------------------------------------------------------------------------------------ GEMM
-constexpr int kTS = 40; // LDS row stride (elements) of a 32-deep k chunk, padded against bank conflicts
-
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs a) {
-  __shared__ __attribute__((aligned(16))) unsigned short As[64 * kTS];
-  __shared__ __attribute__((aligned(16))) unsigned short Bs[64 * kTS];
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-  const int kb = blockIdx.z * a.k_chunk;
-  const int ke = min(a.K, kb + a.k_chunk);
-  const int wm = wave >> 1, wn = wave & 1;
-  const int lr = t >> 2, lk = (t & 3) * 8; // staging: row lr of the tile, k offset lk
-  floatx16 acc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  for (int k0 = kb; k0 < ke; k0 += 32) {
-    {
-      const int m = m0 + lr;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int k = k0 + lk + q;
-        As[lr * kTS + lk + q] = (m < a.M && k < ke) ? a.A[m * a.sam + k * a.sak] : (unsigned short)0;
-      }
-      const int n = n0 + lr;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int k = k0 + lk + q;
-        Bs[lr * kTS + lk + q] = (n < a.N && k < ke) ? a.B[k * a.sbk + n * a.sbn] : (unsigned short)0;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < 32; ks += 16) {
-      const int kk = ks + 8 * (lane >> 5);
-      const shortx8 av = *reinterpret_cast<const shortx8 *>(&As[(wm * 32 + (lane & 31)) * kTS + kk]);
-      const shortx8 bv = *reinterpret_cast<const shortx8 *>(&Bs[(wn * 32 + (lane & 31)) * kTS + kk]);
-      acc = mfma(av, bv, acc);
-    }
-    __syncthreads();
-  }
-  const int n = n0 + wn * 32 + (lane & 31);
-  if (n >= a.N) return;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-    if (m >= a.M) continue;
-    const float v = acc[r];
-    if (a.ep == kEpFwdHidden) {
-      const float z = v + a.bias[n];
-      a.C[m * a.ldc + n] = z;
-      a.Cb[m * a.ldcb + n] = f2bf(a.act == kActGelu ? act<kActGelu>(z) : act<kActHardSwish>(z));
-    } else if (a.ep == kEpFwdOut) {
-      a.C[m * a.ldc + n] = v + a.bias[n];
-    } else if (a.ep == kEpBwdData) {
-      const float z = a.zprev[m * a.ldz + n];
-      a.Cb[m * a.ldcb + n] = f2bf(v * (a.act == kActGelu ? act_grad<kActGelu>(z) : act_grad<kActHardSwish>(z)));
-    } else {
-      atomicAdd(&a.C[m * a.ldc + n], v);
-    }
-  }
-}
-
+// ------------------------------------------------------------------------------------------------ training
 __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
   x += 0x9E3779B97F4A7C15ull;
   x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -128,72 +67,315 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
   return x ^ (x >> 31);
 }
 
-__global__ void k_gather(const float *X, const float *Y, long n, unsigned long long seed, long step, int B,
-                         unsigned short *H0, float *Yb) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= B) return;
-  const long idx = seed ? (long)(mix64(seed ^ mix64((unsigned long long)step * 0x100000001B3ull + i)) % n) : i;
+// A training step is three launches.  One layer's product on 8192 rows is 0.27 GFLOP, a quarter of a microsecond of
+// the matrix cores, so launches and memory round trips between layers were all of the time: as 32 launches with each
+// layer's activations, pre-activations and gradients through memory a step took 658 us (15 products at 33 us, the
+// column sums of the biases at 31 us, ten Adam launches).  Three kernels take 21 + 11 + 5 us, 47 us a step in a row:
+//   k_train_tile  32 rows through all layers and back: activations in LDS, pre-activations in registers
+//   k_train_grad  the weight gradients, which contract over all rows, in up to 16 (above 16384 rows 64) chunks
+//   k_train_adam  sums the chunks in order (no atomics: the same inputs give the same step) and updates everything
+//
+// A work-group's four waves share 32 rows; wave w computes neurons 32 w .. 32 w + 31 of each hidden layer, transposed
+// (out^T = W^T h^T): the weight fragments come straight from the caches (120 KB for the whole network), the activations
+// from LDS, [row][neuron] with a stride of 136 against bank conflicts.  Lane (row, h) then holds 16 neurons of its row.
+constexpr int kTS = 136;
+
+__device__ __forceinline__ shortx8 frag(const unsigned short *p) { return *reinterpret_cast<const shortx8 *>(p); }
+
+// Neuron of accumulator register r within its 32-block, for lane half h.
+__device__ __forceinline__ int acc_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
+
+// Place of element (row r, depth k) in the weights as training reads them: blocks of 32 rows x 16 depths, each one MFMA
+// operand, 1 KB in one piece (with row-major weights, 32 pieces 256 B apart, the kernel takes 26 us instead of 21).
+__device__ __forceinline__ int weight_at(int r, int k, int depth) { return ((r >> 5) * (depth >> 4) + (k >> 4)) * 512 + (r & 31) * 16 + (k & 15); }
+
+// The operands of rows 32 block .. of a 128-deep layer.
+__device__ __forceinline__ void load_layer(shortx8 (&f)[8], const unsigned short *w, int block, int lane) {
 #pragma unroll
-  for (int f = 0; f < 16; ++f) H0[(long)i * 16 + f] = f < kMlpIn ? f2bf(X[idx * kMlpIn + f]) : (unsigned short)0;
-#pragma unroll
-  for (int o = 0; o < kMlpOut; ++o) Yb[(long)i * kMlpOut + o] = Y[idx * kMlpOut + o];
+  for (int ks = 0; ks < 8; ++ks) f[ks] = frag(&w[(block * 8 + ks) * 512 + (lane & 31) * 16 + 8 * (lane >> 5)]);
 }
 
-__global__ __launch_bounds__(256) void k_loss(const float *out, const float *Yb, int B, unsigned short *G,
-                                              float *loss) {
-  __shared__ float part[4];
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const float inv = 1.0f / (float)((long)B * kMlpOut);
-  float sq = 0.0f;
-  if (i < (long)B * kMlpOut) {
-    const float d = out[i] - Yb[i];
-    G[i] = f2bf(2.0f * d * inv);
-    sq = d * d * inv;
+// Their product with the LDS rows.
+__device__ __forceinline__ floatx16 layer128(const shortx8 (&f)[8], const unsigned short *act, int lane) {
+  floatx16 acc = {};
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) acc = mfma(f[ks], frag(&act[(lane & 31) * kTS + 16 * ks + 8 * (lane >> 5)]), acc);
+  return acc;
+}
+
+// Place of (neuron, batch row) in HT and GT: blocks of 32 neurons x 16 rows, so that a wave's MFMA operand (32 neurons,
+// 16 rows, eight rows per lane) is 1 KB in one piece.  With the rows of a neuron contiguous over the whole batch the
+// operand is 32 pieces 16 KB apart; measured no different at 8192 rows, where the wait
+// and not the number of requests counts.
+__device__ __forceinline__ long batch_at(int n, long m, long ld) {
+  return ((long)(n >> 5) * (ld >> 4) + (m >> 4)) * 512 + (n & 31) * 16 + (m & 15);
+}
+
+// 16 values of a lane's row as BF16: neurons n0 + acc_row(r, h) into LDS (row-major) and into HT or GT.
+__device__ __forceinline__ void put_rows(const float (&v)[16], unsigned short *lds, unsigned short *gl, long ld, long m,
+                                         int n0, int lane) {
+  const int row = lane & 31, h = lane >> 5;
+  unsigned short *g = gl ? gl + batch_at(n0, m, ld) : nullptr; // n0 is a multiple of 32
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    unsigned short b[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      b[e] = f2bf(v[4 * q + e]);
+      if (g) g[acc_row(4 * q + e, h) * 16] = b[e];
+    }
+    if (lds)
+      *reinterpret_cast<uint2 *>(&lds[row * kTS + n0 + 8 * q + 4 * h]) =
+          make_uint2((unsigned)b[0] | (unsigned)b[1] << 16, (unsigned)b[2] | (unsigned)b[3] << 16);
   }
-  for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sq;
+}
+
+template<int ACT>
+__global__ __launch_bounds__(256) void k_train_tile(TrainArgs a) {
+  __shared__ __attribute__((aligned(16))) unsigned short buf[2][kTrainRows * kTS]; // activations, then gradients
+  __shared__ __attribute__((aligned(16))) unsigned short small[kTrainRows * 24];   // features, then output gradients
+  __shared__ __attribute__((aligned(16))) float bias[4][kMlpHidden];
+  __shared__ long rows[kTrainRows];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, row = lane & 31, h = lane >> 5, n0 = 32 * wave;
+  // Every weight, bias and target this wave will use is read before anything is written: a load that follows the stores
+  // of a layer's values waits for them as well.  The weights are 232 registers of the one wave per SIMD.
+  const shortx8 f0 = frag(&a.wf[0][wave * 512 + row * 16 + 8 * h]);
+  shortx8 f1[8], f2[8], f3[8], f4[8], g3[8], g2[8], g1[8], g4 = {};
+  load_layer(f1, a.wf[1], wave, lane);
+  load_layer(f2, a.wf[2], wave, lane);
+  load_layer(f3, a.wf[3], wave, lane);
+  load_layer(f4, a.wf[4], 0, lane);
+  if (a.Y) {
+    g4 = frag(&a.wb[4][wave * 512 + row * 16 + 8 * h]);
+    load_layer(g3, a.wb[3], wave, lane);
+    load_layer(g2, a.wb[2], wave, lane);
+    load_layer(g1, a.wb[1], wave, lane);
+  }
+  for (int q = t; q < 4 * kMlpHidden; q += 256) bias[q / kMlpHidden][q % kMlpHidden] = a.bias[q / kMlpHidden][q % kMlpHidden];
+  const long m0 = (long)blockIdx.x * kTrainRows, m = m0 + row;
+  if (t < kTrainRows) {
+    const long i = m0 + t;
+    rows[t] = i >= a.B ? -1 : a.seed ? (long)(mix64(a.seed ^ mix64((unsigned long long)a.step * 0x100000001B3ull + i)) % a.n) : i;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(loss, part[0] + part[1] + part[2] + part[3]);
-}
-
-__device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float((unsigned)h << 16); }
-
-// 256 threads: column n = t % 128, rows b0 + t / 128 + 2q of a 256-row chunk.
-__global__ __launch_bounds__(256) void k_colsum(const unsigned short *G, int B, int N, long ldg, float *db) {
-  const int n = threadIdx.x & 127;
-  if (n >= N) return;
-  const int b0 = blockIdx.x * 256 + (threadIdx.x >> 7);
-  float s = 0.0f;
-  for (int q = 0; q < 128; ++q) {
-    const int b = b0 + 2 * q;
-    if (b < B) s += bf2f(G[(long)b * ldg + n]);
+  const long src = rows[row];
+  float by[8]; // output biases and targets of this lane's row
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int j = acc_row(r, h);
+    by[r] = j < kMlpOut ? a.bias[4][j] : 0.0f;
   }
-  atomicAdd(&db[n], s);
+  float y[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int j = acc_row(r, h);
+    y[r] = a.Y && j < kMlpOut && src >= 0 ? a.Y[src * kMlpOut + j] : 0.0f;
+  }
+  for (int q = t; q < kTrainRows * 16; q += 256) {
+    const int r = q >> 4, f = q & 15;
+    const unsigned short x = f < kMlpIn && rows[r] >= 0 ? f2bf(a.X[rows[r] * kMlpIn + f]) : (unsigned short)0;
+    small[r * 24 + f] = x;
+    if (a.Y && f < kMlpIn) a.HT[0][batch_at(f, m0 + r, a.ld)] = x;
+  }
+  __syncthreads();
+  float z[4][16];
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    floatx16 acc = {};
+    if (l == 0) acc = mfma(f0, frag(&small[row * 24 + 8 * h]), acc);
+    else acc = layer128(l == 1 ? f1 : (l == 2 ? f2 : f3), buf[(l - 1) & 1], lane);
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      z[l][r] = acc[r] + bias[l][n0 + acc_row(r, h)];
+      v[r] = act<ACT>(z[l][r]);
+    }
+    put_rows(v, buf[l & 1], a.Y ? a.HT[l + 1] : nullptr, a.ld, m, n0, lane);
+    __syncthreads();
+  }
+  // the 10 outputs: every wave forms the one 32-neuron block, wave 0 writes it
+  {
+    const floatx16 acc = layer128(f4, buf[1], lane);
+    if (!a.Y) {
+      if (wave == 0 && src >= 0)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int j = acc_row(r, h);
+          if (j < kMlpOut) a.out[m * kMlpOut + j] = acc[r] + by[r];
+        }
+      return;
+    }
+    if (wave == 0) {
+      const float inv = 1.0f / (float)((long)a.B * kMlpOut);
+      float sq = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) { // outputs 0 .. 15
+        const int j = acc_row(r, h);
+        float d = 0.0f;
+        if (j < kMlpOut && src >= 0) d = acc[r] + by[r] - y[r];
+        const unsigned short g = f2bf(2.0f * d * inv);
+        small[row * 24 + j] = g;
+        if (j < kMlpOut) a.GT[4][batch_at(j, m, a.ld)] = g;
+        sq += d * d * inv;
+      }
+      for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+      if (lane == 0) a.loss_part[blockIdx.x] = sq;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int l = 3; l >= 0; --l) {
+    floatx16 acc = {};
+    if (l == 3) acc = mfma(g4, frag(&small[row * 24 + 8 * h]), acc);
+    else acc = layer128(l == 2 ? g3 : (l == 1 ? g2 : g1), buf[(l + 1) & 1], lane);
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = acc[r] * act_grad<ACT>(z[l][r]);
+    put_rows(v, l ? buf[l & 1] : nullptr, a.GT[l], a.ld, m, n0, lane);
+    if (l) __syncthreads();
+  }
 }
 
-__global__ void k_adam(float *p, float *m, float *v, const float *g, long n, float lr, float b1, float b2, float eps,
-                       float c1, float c2, unsigned short *wt, int K, int N, int Kp) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  p[i] = pi;
-  if (wt) wt[(i % N) * Kp + i / N] = f2bf(pi);
+// dW_l = H_l^T G_l and db_l = sum of G_l over the rows of one chunk of the batch.  A work-group takes a 32 x 64 tile of
+// one layer (32 x 32 in the 10-wide last one): 30 tiles.  Its four waves take every fourth 128 rows of the chunk, whose
+// 24 operands are all requested before the first product (they come from other XCDs' caches, about 2 us away: one wave
+// walking 512 rows four operands at a time took 18 us), and are summed in order through LDS.  The bias gradient is one
+// more product, with ones in the place of H.
+constexpr int kGradTiles = 30, kGradRows = 128;
+
+__global__ __launch_bounds__(256) void k_train_grad(TrainArgs a, int chunk_rows, float *__restrict__ part) {
+  __shared__ float sum[4][64][33]; // [wave][lane][register], 16 + 16 of the tile and the bias
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int chunk = blockIdx.x / kGradTiles, tile = blockIdx.x % kGradTiles;
+  int l, kb, nb;
+  if (tile < 24) {
+    l = 1 + tile / 8;
+    kb = (tile % 8) / 2;
+    nb = 2 * (tile % 2);
+  } else if (tile < 26) {
+    l = 0;
+    kb = 0;
+    nb = 2 * (tile - 24);
+  } else {
+    l = 4;
+    kb = tile - 26;
+    nb = 0;
+  }
+  const int i = lane & 31, h = lane >> 5;
+  const bool two = l < 4, bias = kb == 0;
+  const long padded = (a.B + kTrainRows - 1) / kTrainRows * kTrainRows;
+  const long r0 = (long)chunk * chunk_rows, r1 = min(r0 + chunk_rows, padded);
+  // operand of 16 batch rows r ..: 512 values from batch_at(32 kb, r)
+  const unsigned short *H = a.HT[l] + batch_at(32 * kb, 0, a.ld) + i * 16 + 8 * h;
+  const unsigned short *G0 = a.GT[l] + batch_at(32 * nb, 0, a.ld) + i * 16 + 8 * h, *G1 = two ? G0 + 32 * a.ld : G0;
+  const shortx8 ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80}, none = {};
+  floatx16 c0 = {}, c1 = {}, b0 = {}, b1 = {};
+  for (long r = r0 + wave * kGradRows; r < r1; r += 4 * kGradRows) {
+    shortx8 x[8], g0[8], g1[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const bool in = r + 16 * q < r1;
+      x[q] = in ? frag(H + 32 * (r + 16 * q)) : none;
+      g0[q] = in ? frag(G0 + 32 * (r + 16 * q)) : none;
+      g1[q] = in ? frag(G1 + 32 * (r + 16 * q)) : none;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      c0 = mfma(x[q], g0[q], c0);
+      c1 = mfma(x[q], g1[q], c1);
+      if (bias) {
+        b0 = mfma(ones, g0[q], b0);
+        b1 = mfma(ones, g1[q], b1);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    sum[wave][lane][r] = c0[r];
+    sum[wave][lane][16 + r] = c1[r];
+  }
+  sum[wave][lane][32] = h == 0 ? b0[0] : b1[0]; // every row of the bias products is the column sum
+  __syncthreads();
+  float *out = part + (long)chunk * kMlpParams;
+  const int K = l == 0 ? kMlpIn : kMlpHidden, N = l == 4 ? kMlpOut : kMlpHidden;
+  // flat offset of layer l: the layers 1 .. 3 are alike
+  const int ow = l == 0 ? 0 : mlp_offset(1, false) + (l - 1) * (kMlpHidden * kMlpHidden + kMlpHidden), ob = ow + K * N;
+  auto total = [&](int at, int r) { return ((sum[0][at][r] + sum[1][at][r]) + sum[2][at][r]) + sum[3][at][r]; };
+  // register r of lane (i, h) is row acc_row(r % 16, h) and column i (+ 32 for r >= 16); wave w writes registers 8 w ..
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int r = 8 * wave + q, k = 32 * kb + acc_row(r & 15, h), n = 32 * nb + i + (r < 16 ? 0 : 32);
+    if (k < K && n < N && (r < 16 || two)) out[ow + k * N + n] = total(lane, r);
+  }
+  if (bias && wave == 0) {
+    const int n = 32 * nb + i + (h == 0 ? 0 : 32);
+    if (n < N && (h == 0 || two)) out[ob + n] = total(lane, 32);
+  }
 }
 
-__global__ void k_to_bf16t(const float *W, int K, int N, int Kp, unsigned short *wt) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)K * N) return;
-  wt[(i % N) * Kp + i / N] = f2bf(W[i]);
+// Layer and position of flat parameter i; false for a bias.
+__device__ __forceinline__ bool weight_of(int i, int &l, int &k, int &n) {
+  constexpr int hidden = kMlpHidden * kMlpHidden + kMlpHidden, o1 = mlp_offset(1, false), o4 = mlp_offset(4, false);
+  int at;
+  if (i < o1) {
+    l = 0;
+    at = i;
+  } else if (i < o4) {
+    l = 1 + (i - o1) / hidden;
+    at = (i - o1) % hidden;
+  } else {
+    l = 4;
+    at = i - o4;
+  }
+  const int N = l == 4 ? kMlpOut : kMlpHidden, K = l == 0 ? kMlpIn : kMlpHidden;
+  k = at / N;
+  n = at % N;
+  return at < K * N;
 }
 
-__global__ void k_fill(float *p, long n, float v) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
+__device__ __forceinline__ void put_weight(const WeightCopies &c, int l, int k, int n, float w) {
+  const unsigned short b = f2bf(w);
+  const int Kp = l == 0 ? 16 : kMlpHidden;
+  c.wt[l][n * Kp + k] = b;
+  c.wf[l][weight_at(n, k, Kp)] = b;
+  if (l) c.wb[l][weight_at(k, n, l == 4 ? 16 : kMlpHidden)] = b;
+}
+
+__global__ __launch_bounds__(256) void k_train_adam(AdamArgs a) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (a.loss && blockIdx.x == 0 && threadIdx.x < 64) {
+    float s = 0.0f;
+    for (int q = threadIdx.x; q < a.loss_parts; q += 64) s += a.loss_part[q];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (threadIdx.x == 0) *a.loss = s;
+  }
+  if (i >= kMlpParams) return;
+  float g = 0.0f;
+  for (int c = 0; c < a.chunks; c += 16) {
+    float q[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) q[e] = c + e < a.chunks ? a.part[(long)(c + e) * kMlpParams + i] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) g += q[e];
+  }
+  if (a.grads) {
+    a.grads[i] = g;
+    return;
+  }
+  const float mi = a.b1 * a.m[i] + (1.0f - a.b1) * g;
+  const float vi = a.b2 * a.v[i] + (1.0f - a.b2) * g * g;
+  a.m[i] = mi;
+  a.v[i] = vi;
+  const float w = a.p[i] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+  a.p[i] = w;
+  int l, k, n;
+  if (weight_of(i, l, k, n)) put_weight(a.w, l, k, n, w);
+}
+
+__global__ __launch_bounds__(256) void k_pack_weights(const float *p, WeightCopies w) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  int l, k, n;
+  if (i < kMlpParams && weight_of(i, l, k, n)) put_weight(w, l, k, n, p[i]);
 }
 
 // ---------------------------------------------------------------------------------------- fused inference
@@ -639,52 +821,38 @@ inline unsigned grid1(long n, int t) { return (unsigned)((n + t - 1) / t); }
 
 } // namespace
 
-hipError_t launch_gemm(const GemmArgs &a, hipStream_t s) {
-  if (a.M <= 0 || a.N <= 0 || a.K <= 0) return hipSuccess;
-  if (a.k_chunk <= 0 || a.k_chunk % 32) return hipErrorInvalidValue;
-  const int zs = (a.K + a.k_chunk - 1) / a.k_chunk;
-  if (zs > 1 && a.ep != kEpAtomic) return hipErrorInvalidValue;
-  dim3 grid((a.M + 63) / 64, (a.N + 63) / 64, zs);
-  k_gemm<<<grid, 256, 0, s>>>(a);
+hipError_t launch_train_tile(const TrainArgs &a, hipStream_t s) {
+  if (a.B <= 0) return hipSuccess;
+  if (a.n <= 0 || (a.Y && a.ld % 16)) return hipErrorInvalidValue;
+  const unsigned g = (a.B + kTrainRows - 1) / kTrainRows;
+  if (a.act == kActGelu) k_train_tile<kActGelu><<<g, 256, 0, s>>>(a);
+  else k_train_tile<kActHardSwish><<<g, 256, 0, s>>>(a);
   return hipGetLastError();
 }
 
-hipError_t launch_gather(const float *X, const float *Y, long n, unsigned long long seed, long step, int B,
-                         unsigned short *H0, float *Yb, hipStream_t s) {
-  if (B <= 0) return hipSuccess;
-  if (n <= 0) return hipErrorInvalidValue;
-  k_gather<<<grid1(B, 256), 256, 0, s>>>(X, Y, n, seed, step, B, H0, Yb);
+// Rows of a chunk: 16 chunks (480 work-groups, about two per CU) up to 16384 rows, which each wave walks in at most two
+// rounds of 128; 64 above.
+static int chunk_rows(int B) {
+  const int most = train_max_chunks(B);
+  const int r = ((B + most - 1) / most + kTrainRows - 1) / kTrainRows * kTrainRows;
+  return r < 64 ? 64 : r;
+}
+
+int train_chunks(int B) { return (B + chunk_rows(B) - 1) / chunk_rows(B); }
+
+hipError_t launch_train_grad(const TrainArgs &a, float *part, hipStream_t s) {
+  const int chunks = train_chunks(a.B);
+  k_train_grad<<<chunks * kGradTiles, 256, 0, s>>>(a, chunk_rows(a.B), part);
   return hipGetLastError();
 }
 
-hipError_t launch_loss(const float *out, const float *Yb, int B, unsigned short *G, float *loss, hipStream_t s) {
-  if (B <= 0) return hipSuccess;
-  k_loss<<<grid1((long)B * kMlpOut, 256), 256, 0, s>>>(out, Yb, B, G, loss);
+hipError_t launch_train_adam(const AdamArgs &a, hipStream_t s) {
+  k_train_adam<<<(kMlpParams + 255) / 256, 256, 0, s>>>(a);
   return hipGetLastError();
 }
 
-hipError_t launch_colsum(const unsigned short *G, int B, int N, long ldg, float *db, hipStream_t s) {
-  if (B <= 0) return hipSuccess;
-  if (N > 128) return hipErrorInvalidValue;
-  k_colsum<<<grid1(B, 256), 256, 0, s>>>(G, B, N, ldg, db);
-  return hipGetLastError();
-}
-
-hipError_t launch_adam(float *p, float *m, float *v, const float *g, long n, float lr, float b1, float b2, float eps,
-                       float c1, float c2, unsigned short *wt, int K, int N, int Kp, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  k_adam<<<grid1(n, 256), 256, 0, s>>>(p, m, v, g, n, lr, b1, b2, eps, c1, c2, wt, K, N, Kp);
-  return hipGetLastError();
-}
-
-hipError_t launch_to_bf16t(const float *W, int K, int N, int Kp, unsigned short *wt, hipStream_t s) {
-  k_to_bf16t<<<grid1((long)K * N, 256), 256, 0, s>>>(W, K, N, Kp, wt);
-  return hipGetLastError();
-}
-
-hipError_t launch_fill(float *p, long n, float v, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  k_fill<<<grid1(n, 256), 256, 0, s>>>(p, n, v);
+hipError_t launch_pack_weights(const float *p, const WeightCopies &w, hipStream_t s) {
+  k_pack_weights<<<(kMlpParams + 255) / 256, 256, 0, s>>>(p, w);
   return hipGetLastError();
 }
 

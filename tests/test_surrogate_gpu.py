@@ -82,6 +82,31 @@ def test_gradients_match_oracle(net):
         assert rel(gb, rb) < 1e-2 and cosine(gb, rb) > 0.9999, l
 
 
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 500, 1025, 16385, 20000])
+def test_gradients_at_batch_edges(n):
+    """Batches around the 32-row tiles, the 64-row chunks of the weight gradients and the change to smaller chunks
+    above 16384 rows, after a larger batch has used the same arrays; the chunks are summed in order, so a second call
+    gives the same bits."""
+    s = corefl.Surrogate(batch_capacity=max(n, 40) + 7)
+    s.set_activation(corefl.Surrogate.ACT_GELU)
+    params = M.init_params(6)
+    params = [(W, b + 0.05 * np.arange(b.size) / b.size) for W, b in params]
+    s.set_params(params)
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((max(n, 40) + 7, 12)).astype(np.float32)
+    Y = rng.standard_normal((X.shape[0], 10)).astype(np.float32)
+    s.grad(X, Y)
+    loss, g = s.grad(X[:n], Y[:n])
+    again = s.grad(X[:n], Y[:n])
+    loss_ref, ref = M.loss_and_grads([(W.astype(np.float32).astype(np.float64), b.astype(np.float32).astype(np.float64))
+                                      for W, b in params], X[:n].astype(np.float64), Y[:n].astype(np.float64), kind="gelu")
+    assert again[0] == loss and abs(loss - loss_ref) / loss_ref < 1e-4
+    for (gW, gb), (aW, ab), (rW, rb) in zip(g, again[1], ref):
+        assert np.array_equal(gW, aW) and np.array_equal(gb, ab)
+        assert rel(gW, rW) < 1e-2 and cosine(gW, rW) > 0.9999
+        assert rel(gb, rb) < 1e-2 and cosine(gb, rb) > 0.9999
+
+
 def test_adam_step_matches_oracle():
     s = corefl.Surrogate(batch_capacity=256)
     params = M.init_params(6)
