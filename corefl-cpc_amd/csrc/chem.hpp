@@ -8,6 +8,17 @@ namespace corefl {
 
 constexpr int kMaxSpec = 16, kMaxReac = 48, kMaxElem = 8, kMaxSide = 4;
 
+// What a source evaluation reads of one reaction, in 128 consecutive bytes: read array by array a reaction is some
+// twenty scalar loads from as many cache lines, more lines than the scalar cache holds for a mechanism.
+struct ReacRecord {
+  double A, b, Ea, A2, b2, Ea2, troe[4];
+  int type, rev, iorder, n_sides;      // n_sides: distinct species on the left, and on the right times 256
+  unsigned fsp, bsp;                   // their indices, a byte each
+  unsigned long long fnu, bnu;         // and coefficients, 16 bits each
+  unsigned umask, amask;
+};
+static_assert(sizeof(ReacRecord) == 128, "one reaction in two 64-byte scalar loads");
+
 // Plain data, copied to device memory once and read uniformly by every lane.
 struct ChemMech {
   int ns, nr, ne;
@@ -35,6 +46,14 @@ struct ChemMech {
   unsigned umask[kMaxReac], amask[kMaxReac];
   int iorder[kMaxReac];
   double dnu[kMaxReac][kMaxSpec];
+  // the same reactions as the one-lane source walks them, one record each; the order in which the cooperative kernel's
+  // lanes take them (fall-off reactions last, so that a pass of 16 holds either kind), and the most species on a side
+  ReacRecord rec[kMaxReac];
+  int by_cost[kMaxReac], max_f, max_b;
+  // fit ranges common to all species (common_range = 1), so that a wavefront whose temperatures lie on one side of the
+  // middle reads one set of coefficients through scalar loads
+  int common_range;
+  double ct_low, ct_mid, ct_high, c_ln_low, c_ln_high, c_inv_low, c_inv_high;
   int comp[kMaxSpec][kMaxElem];  // element composition
   char species[kMaxSpec][16];
   char elements[kMaxElem][4];

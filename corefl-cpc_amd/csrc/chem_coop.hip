@@ -7,14 +7,20 @@
 // values and row a of the matrix) and reactions a, a + 16, ...: the reaction rates of a source evaluation
 // are computed side by side, each species row accumulates its production terms and Jacobian row, and the LU
 // factorisation and the solves run row-parallel.  Values are exchanged within the row by DPP broadcasts
-// (row_newbcast, a constant source lane), by ds_bpermute for the data-dependent pivot row, and through a
+// (row_newbcast, a constant source lane), by ds_bpermute for a data-dependent pivot row, and through a
 // small per-row LDS area for the rates and concentrations that the reaction lanes read at per-lane indices.
 //
-// Every floating-point operation of the one-lane attempt (chem_kernels.hip) is performed here with the same
-// operands in the same order: the right-looking row-parallel elimination applies to each matrix entry the
-// same updates, in the same order, as the one-lane Doolittle form, and every sum over species is formed in
-// ascending species order from broadcast copies.  The two kernels therefore agree to the last bit where the
-// compiler contracts the same products into FMAs.
+// The chain of one cell is latency: what counts is how long one instruction waits for the one before it.  So the
+// mechanism lives in LDS, laid out so that a lane finds its reaction's or species' values at its own index (read from
+// memory through per-lane and scalar loads, an attempt spent most of its 57 us on them); production terms are dense
+// sums over the reactions, since a lane has nothing better to do; fall-off reactions share the last pass of 16, so that
+// the other passes skip their exponentials; the temperature iteration runs on the mixture's own fit; rows are exchanged
+// only where some cell pivots; and the four stages are one loop, so that the code stays in the instruction cache.
+// An attempt of a wave takes 25 us alone on its SIMD and 37 us with a second one: the three sources 16, of which the
+// Jacobian 2.5, the factorisation 2, the solves 2.3, the temperatures 3.5.
+//
+// The operations are those of the one-lane attempt (chem_kernels.hip) in another order of summation: the two agree to
+// rounding.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -50,11 +56,6 @@ template<int B, int E, class F> __device__ __forceinline__ void static_for(F &&f
   }
 }
 
-// all[l] = lane l's x, l < NS
-template<int NS> __device__ __forceinline__ void row_gather(double x, double *all) {
-  static_for<0, NS>([&](auto L) { all[decltype(L)::value] = row_bcast_c<decltype(L)::value>(x); });
-}
-
 // Orders the LDS traffic of one wavefront: stores before this point are seen by loads after it.
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -62,116 +63,181 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Species thermo tables in LDS, [field][species], read at per-lane species indices.
-struct SpeciesLds {
+constexpr int kPad = 16; // species index of an unused place on a reaction's side: concentration 1, g 0
+
+// The mechanism in LDS.  Species tables [field][species], reaction tables [field][place] and [place][species], places in
+// the order of ChemMech::by_cost.
+struct MechLds {
   double lo[7][kMaxSpec], hi[7][kMaxSpec];
   double t_low[kMaxSpec], t_mid[kMaxSpec], t_high[kMaxSpec];
   double ln_t_low[kMaxSpec], ln_t_high[kMaxSpec], inv_t_low[kMaxSpec], inv_t_high[kMaxSpec];
   double mw[kMaxSpec], imw[kMaxSpec];
+  double A[kMaxReac], b[kMaxReac], Ea[kMaxReac], A2[kMaxReac], b2[kMaxReac], Ea2[kMaxReac], troe[4][kMaxReac];
+  double tb[kMaxSpec][kMaxReac];
+  double dnu[kMaxReac][kMaxSpec], nf[kMaxReac][kMaxSpec], nb[kMaxReac][kMaxSpec];
+  int type[kMaxReac], rev[kMaxReac], iorder[kMaxReac];
+  unsigned fsp[kMaxReac], bsp[kMaxReac];
+  unsigned long long fnu[kMaxReac], bnu[kMaxReac];
 };
 
-// Per-row exchange area: concentrations and g/RT written by the species lanes, rates of progress written by
-// the reaction lanes.
-struct RowLds {
-  double c[kMaxSpec], g[kMaxSpec];
-  double q1[kMaxReac], q2[kMaxReac];
-};
-
-// h_a and cp_a of species a (the one-lane h_cp, one species).
-__device__ __forceinline__ void own_h_cp(const SpeciesLds &S, int a, double t, double &h, double &cp) {
-  const double R = kRu * S.imw[a];
-  const bool below = t < S.t_low[a], above = t > S.t_high[a];
-  if (below || above) {
-    const double tt = below ? S.t_low[a] : S.t_high[a];
-    double c[5];
+__device__ __forceinline__ void stage_mechanism(const ChemMech &m, MechLds &S) {
+  for (int i = threadIdx.x; i < kMaxSpec; i += blockDim.x) {
 #pragma unroll
-    for (int q = 0; q < 5; ++q) c[q] = below ? S.lo[q][a] : S.hi[q][a];
-    const double c5 = below ? S.lo[5][a] : S.hi[5][a];
-    const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt;
-    const double cc = c[0] + c[1] * tt + c[2] * tt2 + c[3] * tt3 + c[4] * tt4;
-    const double hh = c[0] * tt + 0.5 * c[1] * tt2 + c[2] * tt3 * kThird + 0.25 * c[3] * tt4 + 0.2 * c[4] * tt5 + c5;
-    h = (hh + cc * (t - tt)) * R;
-    cp = cc * R;
-  } else {
-    const bool use_lo = t < S.t_mid[a];
-    double c[6];
+    for (int q = 0; q < 7; ++q) {
+      S.lo[q][i] = m.lo[i][q];
+      S.hi[q][i] = m.hi[i][q];
+    }
+    S.t_low[i] = m.t_low[i];
+    S.t_mid[i] = m.t_mid[i];
+    S.t_high[i] = m.t_high[i];
+    S.ln_t_low[i] = m.ln_t_low[i];
+    S.ln_t_high[i] = m.ln_t_high[i];
+    S.inv_t_low[i] = m.inv_t_low[i];
+    S.inv_t_high[i] = m.inv_t_high[i];
+    S.mw[i] = m.mw[i];
+    S.imw[i] = m.imw[i];
+  }
+  for (int p = threadIdx.x; p < m.nr; p += blockDim.x) {
+    const int r = m.by_cost[p];
+    const ReacRecord q = m.rec[r];
+    S.A[p] = q.A;
+    S.b[p] = q.b;
+    S.Ea[p] = q.Ea;
+    S.A2[p] = q.A2;
+    S.b2[p] = q.b2;
+    S.Ea2[p] = q.Ea2;
 #pragma unroll
-    for (int q = 0; q < 6; ++q) c[q] = use_lo ? S.lo[q][a] : S.hi[q][a];
-    const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t5 = t4 * t;
-    h = (c[0] * t + 0.5 * c[1] * t2 + c[2] * t3 * kThird + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5]) * R;
-    cp = (c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4) * R;
+    for (int k = 0; k < 4; ++k) S.troe[k][p] = q.troe[k];
+    S.type[p] = q.type;
+    S.rev[p] = q.rev;
+    S.iorder[p] = q.iorder;
+    unsigned f = q.fsp, b = q.bsp;
+    for (int k = q.n_sides & 255; k < kMaxSide; ++k) f |= (unsigned)kPad << 8 * k;
+    for (int k = q.n_sides >> 8; k < kMaxSide; ++k) b |= (unsigned)kPad << 8 * k;
+    S.fsp[p] = f;
+    S.bsp[p] = b;
+    S.fnu[p] = q.fnu; // coefficient 0 in unused places
+    S.bnu[p] = q.bnu;
+  }
+  for (int q = threadIdx.x; q < m.nr * kMaxSpec; q += blockDim.x) {
+    const int p = q / kMaxSpec, n = q % kMaxSpec, r = m.by_cost[p];
+    S.dnu[p][n] = m.dnu[r][n];
+    S.nf[p][n] = m.nf[r][n];
+    S.nb[p][n] = m.nb[r][n];
+    S.tb[n][p] = m.tb[r][n];
   }
 }
 
+// Per-row exchange area: concentrations and g/RT written by the species lanes, rates of progress written by
+// the reaction lanes (q1 the net one where no Jacobian is formed).
+struct RowLds {
+  double c[kMaxSpec + 1], g[kMaxSpec + 1];
+  double q1[kMaxReac], q2[kMaxReac];
+};
+
+// Sum over the row's 16 lanes, the same bits in all of them (each rotation adds two values that both lanes hold).
+template<int N> __device__ __forceinline__ double row_rotate(double x) {
+  int2 v = __builtin_bit_cast(int2, x);
+  v.x = __builtin_amdgcn_update_dpp(0, v.x, 0x120 + N, 0xF, 0xF, false);
+  v.y = __builtin_amdgcn_update_dpp(0, v.y, 0x120 + N, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, v);
+}
+__device__ __forceinline__ double row_sum(double x) {
+  x += row_rotate<8>(x);
+  x += row_rotate<4>(x);
+  x += row_rotate<2>(x);
+  x += row_rotate<1>(x);
+  return x;
+}
+
 // g_a / (R T) of species a (the one-lane gibbs, one species).
-__device__ __forceinline__ double own_gibbs(const SpeciesLds &S, int a, double t, double lnT, double iT) {
+__device__ __forceinline__ double own_gibbs(const MechLds &S, int a, double t, double lnT, double iT) {
   const bool below = t < S.t_low[a], above = t > S.t_high[a];
   const double tt = below ? S.t_low[a] : (above ? S.t_high[a] : t);
   const bool use_lo = below || (!above && t < S.t_mid[a]);
   double c[7];
 #pragma unroll
   for (int q = 0; q < 7; ++q) c[q] = use_lo ? S.lo[q][a] : S.hi[q][a];
-  const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt;
   const double lt = below ? S.ln_t_low[a] : (above ? S.ln_t_high[a] : lnT);
   const double itt = below ? S.inv_t_low[a] : (above ? S.inv_t_high[a] : iT);
-  return c[0] * (1.0 - lt) - 0.5 * c[1] * tt - c[2] * tt2 * kSixth - c[3] * tt3 * kTwelfth - c[4] * tt4 * 0.05 +
-         c[5] * itt - c[6];
+  return gibbs_fit(c, tt, lt, itt);
 }
 
-// Newton temperature at fixed E (the one-lane update_t): yk = this lane's mass fraction (0 beyond NS).
+// Newton temperature at fixed E (the one-lane update_t): yk = this lane's mass fraction (0 beyond NS).  The mixture's
+// enthalpy and heat capacity are those of its summed coefficients where all species share their fit range, else the sums
+// of the species' own.
 template<int NS>
-__device__ __forceinline__ double row_update_t(const ChemMech &m, const SpeciesLds &S, int a, double t, double yk,
-                                               double E) {
-  double y[NS];
-  row_gather<NS>(yk, y);
-  double imw = 0;
-#pragma unroll
-  for (int l = 0; l < NS; ++l) imw += y[l] * m.imw[l];
-  const double R = kRu * imw;
-  double err = 1e+6;
+__device__ __forceinline__ double row_update_t(const ChemMech &m, const MechLds &S, int a, double t, double yk, double E) {
+  const double R = kRu * row_sum(yk * S.imw[a]), yr = yk * (kRu * S.imw[a]);
+  double err = 1e+6, C[6];
+  int side = -1;
+#pragma unroll 1
   for (int it = 0; it < 100 && err > 1e-8; ++it) {
     double h, cp;
-    own_h_cp(S, a, t, h, cp);
-    double hs[NS], cps[NS];
-    row_gather<NS>(h, hs);
-    row_gather<NS>(cp, cps);
-    double cpt = 0, hh = 0;
+    if (m.common_range) {
+      const int now = t < m.ct_mid ? 0 : 1;
+      if (now != side) { // all lanes of a row alike
 #pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      cpt += cps[l] * y[l];
-      hh += hs[l] * y[l];
+        for (int q = 0; q < 6; ++q) C[q] = row_sum(yr * (now ? S.hi[q][a] : S.lo[q][a]));
+        side = now;
+      }
+      h_cp_fit(C, 1.0, t, fmin(fmax(t, m.ct_low), m.ct_high), h, cp);
+    } else {
+      const double lo = S.t_low[a], hi = S.t_high[a], tt = t < lo ? lo : (t > hi ? hi : t);
+      const bool use_lo = t < lo || (!(t > hi) && t < S.t_mid[a]);
+      double c[6];
+#pragma unroll
+      for (int q = 0; q < 6; ++q) c[q] = use_lo ? S.lo[q][a] : S.hi[q][a];
+      h_cp_fit(c, yr, t, tt, h, cp);
+      h = row_sum(h);
+      cp = row_sum(cp);
     }
-    const double t1 = t - (hh - R * t - E) / (cpt - R);
+    const double t1 = t - (h - R * t - E) / (cp - R);
     err = fabs(1 - t1 / t);
     t = t1;
   }
   return t;
 }
 
-// Rates of progress of reaction r at the row's state (the reaction body of the one-lane source).
-__device__ __forceinline__ void reaction_rates(const ChemMech &m, const RowLds &X, int r, int ns, double t,
-                                               double lnT, double iT, double tp, double &q1o, double &q2o) {
-  const int ty = m.type[r];
-  const int nfs = m.nfs[r], nbs = m.nbs[r];
-  double kf = arrhenius(lnT, iT, m.A[r], m.b[r], m.Ea[r]);
+// Rates of progress of the reaction in place r at the row's state (the reaction body of the one-lane source).  (Two
+// places at a time, their exponentials formed together without branches, take as long.)
+__device__ __forceinline__ void reaction_rates(const ChemMech &m, const MechLds &S, const RowLds &X, int r, int ns, double t,
+                                               double lnT, double iT, double &q1o, double &q2o) {
+  const int ty = S.type[r], rev = S.rev[r], order = S.iorder[r];
+  const unsigned fsp = S.fsp[r], bsp = S.bsp[r];
+  const unsigned long long fnu = S.fnu[r], bnu = S.bnu[r];
+  const double A2 = S.A2[r], b2 = S.b2[r], Ea2 = S.Ea2[r];
+  // both sides at once: the sum of nu g and the product of c^nu
+  double dg = 0, q1 = 1.0, q2 = ty != 0 ? 1.0 : 0.0;
+  auto side = [&](unsigned sp, unsigned long long nu, int most, double sign, double &q) {
+    for (int s = 0; s < most; ++s) {
+      const int l = sp >> 8 * s & 255u, n = (short)(nu >> 16 * s & 65535u);
+      const double x = X.c[l];
+      dg += X.g[l] * (sign * n);
+      if (n == 1) q *= x;
+      else q *= int_pow(x, n);
+    }
+  };
+  side(fsp, fnu, m.max_f, -1.0, q1);
+  side(bsp, bnu, m.max_b, 1.0, q2);
+  double kf = arrhenius(lnT, iT, S.A[r], S.b[r], S.Ea[r]);
   double cc = 0;
-  if (ty >= 4) {
-    for (int l = 0; l < ns; ++l) cc += X.c[l] * m.tb[r][l];
-  }
+  if (ty >= 4)
+    for (int l = 0; l < ns; ++l) cc += X.c[l] * S.tb[l][r];
   if (ty == 3) {
-    kf += arrhenius(lnT, iT, m.A2[r], m.b2[r], m.Ea2[r]);
+    kf += arrhenius(lnT, iT, A2, b2, Ea2);
   } else if (ty == 4) {
     kf *= cc;
   } else if (ty > 4) {
-    const double klow = arrhenius(lnT, iT, m.A2[r], m.b2[r], m.Ea2[r]), khigh = kf;
+    const double klow = arrhenius(lnT, iT, A2, b2, Ea2), khigh = kf;
     if (khigh < 1e-25 && klow < 1e-25) {
       kf = 0;
     } else {
       const double pr = klow * cc / khigh;
       double F = 1.0;
       if (ty > 5) {
-        double fc = (1 - m.troe[r][0]) * exp(-t / m.troe[r][1]) + m.troe[r][0] * exp(-t / m.troe[r][2]);
-        if (ty == 7) fc += exp(-m.troe[r][3] / t);
+        double fc = (1 - S.troe[0][r]) * exp(-t / S.troe[1][r]) + S.troe[0][r] * exp(-t / S.troe[2][r]);
+        if (ty == 7) fc += exp(-S.troe[3][r] * iT);
         const double lfc = log10(fc);
         const double cq = -0.4 - 0.67 * lfc, nq = 0.75 - 1.27 * lfc;
         const double lpr = log10(pr);
@@ -182,87 +248,63 @@ __device__ __forceinline__ void reaction_rates(const ChemMech &m, const RowLds &
     }
   }
   double kb = 0;
-  if (ty != 0 && m.rev[r] == 1) {
-    kb = arrhenius(lnT, iT, m.A2[r], m.b2[r], m.Ea2[r]);
+  if (ty != 0 && rev == 1) {
+    kb = arrhenius(lnT, iT, A2, b2, Ea2);
     if (ty == 4) kb *= cc;
   }
   if (m.need_gibbs && ty != 0 && ty != 2) {
-    double dg = 0;
-    for (int s = 0; s < nbs; ++s) dg += X.g[m.bsp[r][s]] * m.bnu[r][s];
-    for (int s = 0; s < nfs; ++s) dg -= X.g[m.fsp[r][s]] * m.fnu[r][s];
-    kb = kf / (int_pow(tp, m.iorder[r]) * exp(-dg));
+    const double tp = kPatm / kRu * 1e-3 * iT, itp = kRu / kPatm * 1e+3 * t;
+    kb = kf * exp(dg) * int_pow(order < 0 ? tp : itp, order < 0 ? -order : order);
   }
-  double q1 = 1.0, q2 = ty != 0 ? 1.0 : 0.0;
-  for (int s = 0; s < nfs; ++s) q1 *= int_pow(X.c[m.fsp[r][s]], m.fnu[r][s]);
-  if (ty != 0)
-    for (int s = 0; s < nbs; ++s) q2 *= int_pow(X.c[m.bsp[r][s]], m.bnu[r][s]);
   q1o = q1 * kf;
   q2o = q2 * kb;
 }
 
-// Chemical source (and with JAC the Jacobian row a) of the row's cell: lane a returns omega_a; yall holds
-// every species' rho Y (replicated).
-template<int NS, bool JAC>
-__device__ __forceinline__ double row_source(const ChemMech &m, const SpeciesLds &S, RowLds &X, int a, int gl,
-                                             double t, double ya, const double *yall, double *Jrow) {
+// Chemical source of the row's cell, lane a omega_a; with jac (uniform) also row a of the Jacobian.  ya is this lane's
+// rho Y.
+template<int NS>
+__device__ __forceinline__ double row_source(const ChemMech &m, const MechLds &S, RowLds &X, int a, int gl, double t, double ya,
+                                             bool jac, double (&Jrow)[NS]) {
   const double lnT = log(t), iT = 1.0 / t;
-  const double tp = kPatm / kRu * 1e-3 / t;
   X.c[gl] = ya * S.imw[a] * 1e-3;
-  if (m.need_gibbs) X.g[gl] = own_gibbs(S, a, t, lnT, iT);
+  X.g[gl] = m.need_gibbs ? own_gibbs(S, a, t, lnT, iT) : 0.0;
   wave_sync();
   const int nr = m.nr;
+#pragma unroll 1
   for (int r0 = 0; r0 < nr; r0 += RW) {
     const int r = r0 + gl;
     if (r < nr) {
       double q1, q2;
-      reaction_rates(m, X, r, NS, t, lnT, iT, tp, q1, q2);
-      X.q1[r] = q1;
+      reaction_rates(m, S, X, r, NS, t, lnT, iT, q1, q2);
+      X.q1[r] = jac ? q1 : q1 - q2;
       X.q2[r] = q2;
     }
   }
   wave_sync();
-  double cr = 0, de = 0;
-  if constexpr (JAC) {
+  const double scale = 1e+3 * S.mw[a];
+  double w = 0;
+  if (!jac) {
+#pragma unroll 8
+    for (int r = 0; r < nr; ++r) w = fma(S.dnu[r][a], X.q1[r], w);
+  } else {
+    // column n of a reaction's term is lane n's, and goes round the row
 #pragma unroll
     for (int n = 0; n < NS; ++n) Jrow[n] = 0;
-  }
-  const unsigned bit = 1u << a;
-  for (int r = 0; r < nr; ++r) {
-    const double q1 = X.q1[r], q2 = X.q2[r];
-    const int nfs = m.nfs[r], nbs = m.nbs[r];
-    for (int s = 0; s < nfs; ++s) {
-      if (m.fsp[r][s] == a) {
-        const double nu = m.fnu[r][s];
-        cr += q2 * nu;
-        de += q1 * nu;
-      }
+#pragma unroll 2
+    for (int r = 0; r < nr; ++r) {
+      const double q1 = X.q1[r], q2 = X.q2[r], dn = S.dnu[r][a];
+      const double v = S.nf[r][a] * q1 - S.nb[r][a] * q2;
+      w = fma(dn, q1 - q2, w);
+      static_for<0, NS>([&](auto N) { Jrow[decltype(N)::value] += dn * row_bcast_c<decltype(N)::value>(v); });
     }
-    for (int s = 0; s < nbs; ++s) {
-      if (m.bsp[r][s] == a) {
-        const double nu = m.bnu[r][s];
-        cr += q1 * nu;
-        de += q2 * nu;
-      }
-    }
-    if constexpr (JAC) {
-      const unsigned um = m.umask[r];
-      if (m.amask[r] & bit) {
-        const double dn = m.dnu[r][a];
-#pragma unroll
-        for (int n = 0; n < NS; ++n)
-          if (um >> n & 1u) Jrow[n] += dn * (m.nf[r][n] * q1 - m.nb[r][n] * q2);
-      }
-    }
-  }
-  if constexpr (JAC) {
-#pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      const double inv = yall[n] > 1e-30 ? 1.0 / yall[n] : 0.0;
-      Jrow[n] = Jrow[n] * inv * (1e+3 * S.mw[a]);
-    }
+    const double inv = ya > 1e-30 ? 1.0 / ya : 0.0;
+    static_for<0, NS>([&](auto N) {
+      constexpr int n = decltype(N)::value;
+      Jrow[n] = Jrow[n] * row_bcast_c<n>(inv) * scale;
+    });
   }
   wave_sync(); // the exchange area is rewritten by the next evaluation
-  return cr * (1e+3 * S.mw[a]) - de * (1e+3 * S.mw[a]);
+  return w * scale;
 }
 
 // Row-parallel LU with partial pivoting of the matrix whose row a is held by lane a.  Leaves L (unit, below
@@ -287,14 +329,18 @@ template<int NS> __device__ __forceinline__ int row_lu(double *row, int a) {
       }
     }
     piv[k] = ik;
-    double prow[NS], krow[NS];
+    double prow[NS];
+    if (__any(ik != k)) {
 #pragma unroll
-    for (int t = 0; t < NS; ++t) {
-      prow[t] = __shfl(row[t], ik, RW);
-      krow[t] = row_bcast_c<k>(row[t]);
+      for (int t = 0; t < NS; ++t) {
+        prow[t] = __shfl(row[t], ik, RW);
+        const double krow = row_bcast_c<k>(row[t]);
+        row[t] = a == k ? prow[t] : (a == ik ? krow : row[t]);
+      }
+    } else {
+#pragma unroll
+      for (int t = k; t < NS; ++t) prow[t] = row_bcast_c<k>(row[t]);
     }
-#pragma unroll
-    for (int t = 0; t < NS; ++t) row[t] = a == k ? prow[t] : (a == ik ? krow[t] : row[t]);
     const double inv = 1.0 / prow[k];
     if (a > k) {
       const double l = row[k] * inv;
@@ -348,56 +394,52 @@ struct RowCell {
 
 // One ROK4E attempt of the row's cell: the one-lane rok4e_attempt, species-parallel.
 template<int NS>
-__device__ __forceinline__ void row_attempt(const ChemMech &m, const SpeciesLds &S, RowLds &X, int a, int gl,
+__device__ __forceinline__ void row_attempt(const ChemMech &m, const MechLds &S, RowLds &X, int a, int gl,
                                             RowCell &s, double rtol, double atol) {
   const bool own = gl < NS; // lanes beyond NS carry zeros
   const double dt = s.dt;
-  double yall[NS], Jrow[NS];
-  row_gather<NS>(s.y, yall);
-  double w = row_source<NS, true>(m, S, X, a, gl, s.T, s.y, yall, Jrow);
+  double Jrow[NS];
   const double rem = dt - s.time;
   const double hs = s.h * kStretch >= rem ? rem : s.h;
-#pragma unroll
-  for (int n = 0; n < NS; ++n) Jrow[n] = -hs * G * Jrow[n];
-#pragma unroll
-  for (int n = 0; n < NS; ++n)
-    if (n == a) Jrow[n] += 1.0;
-  const int src = row_lu<NS>(Jrow, a);
-  const double k1 = row_solve<NS>(Jrow, a, src, w);
   const double irho = 1.0 / s.rho;
-  double ys = s.y + hs * A21 * k1;
-  double Ts = row_update_t<NS>(m, S, a, s.T, own ? ys * irho : 0.0, s.E);
-  row_gather<NS>(ys, yall);
-  w = row_source<NS, false>(m, S, X, a, gl, Ts, ys, yall, nullptr);
-  double k2 = row_solve<NS>(Jrow, a, src, w + G21 * k1);
-  k2 -= G21 * k1;
-  ys = s.y + hs * (A31 * k1 + A32 * k2);
-  Ts = row_update_t<NS>(m, S, a, Ts, own ? ys * irho : 0.0, s.E);
-  row_gather<NS>(ys, yall);
-  w = row_source<NS, false>(m, S, X, a, gl, Ts, ys, yall, nullptr);
-  double k3 = row_solve<NS>(Jrow, a, src, w + G31 * k1 + G32 * k2);
-  k3 -= G31 * k1 + G32 * k2;
-  double k4 = row_solve<NS>(Jrow, a, src, w + G41 * k1 + G42 * k2 + G43 * k3);
-  k4 -= G41 * k1 + G42 * k2 + G43 * k3;
-  const double ynew = s.y + hs * (B1 * k1 + B2 * k2 + B4 * k4);
-  const double dy = hs * (E1 * k1 + E2 * k2 + E3 * k3 + E4 * k4) / (rtol * ynew + atol);
-  double dys[NS];
-  row_gather<NS>(dy, dys);
-  double err = 0;
+  double k1 = 0, k2 = 0, k3 = 0, w = 0, ys = s.y, Ts = s.T, err = 0;
+  int src = 0;
+#pragma unroll 1
+  for (int st = 0; st < 5; ++st) {
+    if (st != 3) { // the fourth stage takes the third's source
+      if (st < 4) ys = s.y + hs * (kStageA[st][0] * k1 + kStageA[st][1] * k2);
+      // st 4: ys is the new state, and an accepted step gets its temperature from the old one
+      if (st > 0 && (st < 4 || err <= 1)) Ts = row_update_t<NS>(m, S, a, st == 4 ? s.T : Ts, own ? ys * irho : 0.0, s.E);
+      if (st == 4) break;
+      w = row_source<NS>(m, S, X, a, gl, Ts, ys, st == 0, Jrow);
+      if (st == 0) {
 #pragma unroll
-  for (int l = 0; l < NS; ++l) err += dys[l] * dys[l];
-  err = sqrt(err / NS);
+        for (int n = 0; n < NS; ++n) Jrow[n] = -hs * G * Jrow[n] + (n == a ? 1.0 : 0.0);
+        src = row_lu<NS>(Jrow, a);
+      }
+    }
+    const double c = kStageG[st][0] * k1 + kStageG[st][1] * k2 + kStageG[st][2] * k3;
+    const double k = row_solve<NS>(Jrow, a, src, w + c) - c;
+    if (st == 0) k1 = k;
+    else if (st == 1) k2 = k;
+    else if (st == 2) k3 = k;
+    else {
+      ys = s.y + hs * (B1 * k1 + B2 * k2 + B4 * k);
+      const double dy = hs * (E1 * k1 + E2 * k2 + E3 * k3 + E4 * k) / (rtol * ys + atol);
+      err = sqrt(row_sum(own ? dy * dy : 0.0) / NS);
+    }
+  }
   double hstar = hs;
-  if (s.steps > 0) hstar *= fmin(5.0, fmax(0.2, 0.8 * pow(s.err_last, 0.1) * pow(err + 1e-20, -0.175)));
+  if (s.steps > 0) hstar *= step_factor(s.err_last, err);
   else if (!(err <= 1)) hstar *= 0.2;
   if (err <= 1 && hs < s.h) hstar = fmax(hstar, s.h);
   s.h = hstar;
   ++s.attempts;
   if (err <= 1) {
-    s.y = own ? ynew : 0.0;
+    s.y = own ? ys : 0.0;
     s.time += hs;
     s.err_last = fmax(err, 1e-30);
-    s.T = row_update_t<NS>(m, S, a, s.T, s.y * irho, s.E);
+    s.T = Ts;
     ++s.steps;
   } else {
     ++s.rejects;
@@ -413,31 +455,22 @@ template<int NS>
 __global__ __launch_bounds__(256) void k_chem_coop(const ChemMech *__restrict__ mp, ChemBatch b, double dt,
                                                    double rtol, double atol, int max_attempts, int *counter,
                                                    int resume) {
-  __shared__ SpeciesLds S;
+  __shared__ MechLds S;
   __shared__ RowLds rows[256 / RW];
+  const int n_work = work_count(b);
+  // work-groups beyond one row per cell would find the queue empty
+  if ((long)blockIdx.x * (blockDim.x / RW) >= n_work) return;
   const ChemMech &m = *mp;
-  for (int i = threadIdx.x; i < kMaxSpec; i += blockDim.x) {
-#pragma unroll
-    for (int q = 0; q < 7; ++q) {
-      S.lo[q][i] = m.lo[i][q];
-      S.hi[q][i] = m.hi[i][q];
-    }
-    S.t_low[i] = m.t_low[i];
-    S.t_mid[i] = m.t_mid[i];
-    S.t_high[i] = m.t_high[i];
-    S.ln_t_low[i] = m.ln_t_low[i];
-    S.ln_t_high[i] = m.ln_t_high[i];
-    S.inv_t_low[i] = m.inv_t_low[i];
-    S.inv_t_high[i] = m.inv_t_high[i];
-    S.mw[i] = m.mw[i];
-    S.imw[i] = m.imw[i];
+  stage_mechanism(m, S);
+  if (threadIdx.x < blockDim.x / RW) {
+    rows[threadIdx.x].c[kPad] = 1.0;
+    rows[threadIdx.x].g[kPad] = 0.0;
   }
   __syncthreads();
   const int lane = __lane_id();
   const int gl = lane & (RW - 1);
   const int a = gl < NS ? gl : 0; // species of this lane (lanes beyond NS mirror species 0 and carry zeros)
   RowLds &X = rows[threadIdx.x / RW];
-  const int n_work = work_count(b);
   RowCell s;
   int cell = -1;
   bool exhausted = false;

@@ -16,46 +16,83 @@ constexpr double kRu = 8314.462618, kPatm = 101325.0;
 // constant divisions of the polynomial fits as products (a few ulp from the divided form)
 constexpr double kThird = 1.0 / 3.0, kSixth = 1.0 / 6.0, kTwelfth = 1.0 / 12.0;
 
-// h_k and cp_k per unit mass, linear extrapolation outside [t_low, t_high] (Thermo.cu:470-520).
-// h and cp of species i at t (the body of h_cp for one species).
-__device__ __forceinline__ void h_cp_one(const ChemMech &m, int i, double t, double &h, double &cp) {
-  const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t5 = t4 * t;
-  const double R = kRu * m.imw[i];
-  const bool below = t < m.t_low[i], above = t > m.t_high[i];
-  if (below || above) {
-    const double tt = below ? m.t_low[i] : m.t_high[i];
-    const double *c = below ? m.lo[i] : m.hi[i];
-    const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt;
-    const double cc = c[0] + c[1] * tt + c[2] * tt2 + c[3] * tt3 + c[4] * tt4;
-    const double hh = c[0] * tt + 0.5 * c[1] * tt2 + c[2] * tt3 * kThird + 0.25 * c[3] * tt4 + 0.2 * c[4] * tt5 + c[5];
-    h = (hh + cc * (t - tt)) * R;
-    cp = cc * R;
-  } else {
-    const double *c = t < m.t_mid[i] ? m.lo[i] : m.hi[i];
-    h = (c[0] * t + 0.5 * c[1] * t2 + c[2] * t3 * kThird + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5]) * R;
-    cp = (c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4) * R;
-  }
+// The mechanism behind a pointer the optimiser cannot see through: its loads stay where they are used.  Hoisted out of
+// the loops around them, a mechanism's hundreds of uniform values overflow the scalar registers, and every use becomes a
+// read from a vector register's lane.
+__device__ __forceinline__ const ChemMech &opaque(const ChemMech *mp) {
+  typedef const __attribute__((address_space(4))) ChemMech *ConstMech;
+  ConstMech mc = (ConstMech)mp;
+  asm volatile("" : "+s"(mc));
+  return *(const ChemMech *)mc;
+}
+
+// Which fit coefficients a wavefront needs: the low ones where every active lane is below the middle of the common fit
+// range, the high ones where every lane is above it, else each lane its own (a flame front, ranges that differ between
+// species, NaN).  On one side the coefficients are uniform scalar loads; lane by lane they are 27 vector loads of 16
+// bytes for the nine species, at 1 wave per SIMD a wait for each.
+enum FitSide { kFitLow, kFitHigh, kFitMixed };
+__device__ __forceinline__ FitSide fit_side(const ChemMech &m, double t) {
+  if (!m.common_range) return kFitMixed;
+  if (__all(t < m.ct_mid)) return kFitLow;
+  if (__all(t >= m.ct_mid)) return kFitHigh;
+  return kFitMixed;
+}
+
+// h_k and cp_k per unit mass (Thermo.cu:470-520): the fit at the temperature clamped to [t_low, t_high], continued
+// linearly outside (inside, the term (t - tt) cp is an exact zero).
+__device__ __forceinline__ void h_cp_fit(const double *c, double R, double t, double tt, double &h, double &cp) {
+  // fused multiply-adds written out: the copies for uniform and for per-lane coefficients round alike
+  const double cc = fma(tt, fma(tt, fma(tt, fma(tt, c[4], c[3]), c[2]), c[1]), c[0]);
+  const double hh = fma(tt, fma(tt, fma(tt, fma(tt, fma(tt, 0.2 * c[4], 0.25 * c[3]), c[2] * kThird), 0.5 * c[1]), c[0]), c[5]);
+  h = fma(cc, t - tt, hh) * R;
+  cp = cc * R;
 }
 
 template<int NS> __device__ __forceinline__ void h_cp(const ChemMech &m, double t, double *h, double *cp) {
+  const FitSide side = fit_side(m, t);
+  if (side != kFitMixed) {
+    const double(*c)[7] = side == kFitLow ? m.lo : m.hi;
+    const double tt = fmin(fmax(t, m.ct_low), m.ct_high);
 #pragma unroll
-  for (int i = 0; i < NS; ++i) h_cp_one(m, i, t, h[i], cp[i]);
+    for (int i = 0; i < NS; ++i) h_cp_fit(c[i], kRu * m.imw[i], t, tt, h[i], cp[i]);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    const double tt = t < m.t_low[i] ? m.t_low[i] : (t > m.t_high[i] ? m.t_high[i] : t);
+    const bool low = t < m.t_low[i] || (!(t > m.t_high[i]) && t < m.t_mid[i]);
+    h_cp_fit(low ? m.lo[i] : m.hi[i], kRu * m.imw[i], t, tt, h[i], cp[i]);
+  }
 }
 
 // g_k / (R T), clamped to the fit range (Thermo.cu:574-598).  lnT = log(t): one logarithm serves every
 // species whose fit range holds t; the logarithms of the range ends are tabulated.
+__device__ __forceinline__ double gibbs_fit(const double *c, double tt, double lt, double itt) {
+  const double p = fma(tt, fma(tt, fma(tt, c[4] * 0.05, c[3] * kTwelfth), c[2] * kSixth), 0.5 * c[1]);
+  return fma(c[0], 1.0 - lt, fma(c[5], itt, -c[6])) - tt * p;
+}
+
 template<int NS>
 __device__ __forceinline__ void gibbs(const ChemMech &m, double t, double lnT, double iT, double *g) {
+  const FitSide side = fit_side(m, t);
+  if (side != kFitMixed) {
+    const double(*c)[7] = side == kFitLow ? m.lo : m.hi;
+    const bool below = t < m.ct_low, above = t > m.ct_high;
+    const double tt = below ? m.ct_low : (above ? m.ct_high : t);
+    const double lt = below ? m.c_ln_low : (above ? m.c_ln_high : lnT);
+    const double itt = below ? m.c_inv_low : (above ? m.c_inv_high : iT);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) g[i] = gibbs_fit(c[i], tt, lt, itt);
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
     const bool below = t < m.t_low[i], above = t > m.t_high[i];
     const double tt = below ? m.t_low[i] : (above ? m.t_high[i] : t);
     const double *c = below ? m.lo[i] : (above ? m.hi[i] : (t < m.t_mid[i] ? m.lo[i] : m.hi[i]));
-    const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt;
     const double lt = below ? m.ln_t_low[i] : (above ? m.ln_t_high[i] : lnT);
     const double itt = below ? m.inv_t_low[i] : (above ? m.inv_t_high[i] : iT);
-    g[i] = c[0] * (1.0 - lt) - 0.5 * c[1] * tt - c[2] * tt2 * kSixth - c[3] * tt3 * kTwelfth - c[4] * tt4 * 0.05 +
-           c[5] * itt - c[6];
+    g[i] = gibbs_fit(c, tt, lt, itt);
   }
 }
 
@@ -77,51 +114,60 @@ __device__ __forceinline__ double int_pow(double x, int k) {
 // Chemical source omega [kg/(m^3 s)] of one cell (FiniteRateChem.cu:1466-1605).  With JAC, also the
 // Jacobian d omega / d(rho Y) with the rates of progress frozen (ConstVolumeReactor.cpp:1168-1187); columns of
 // species with rho Y at or below floor are zero (1e-30 in the reactor, 1e-25 in Wu's EPI, StrangSplitting.cu:164).
-// Stoichiometry is walked through each reaction's species lists (a few entries) rather than all species;
-// the Jacobian keeps static indices (register-resident) and skips rows and columns through the reaction's
-// species bit masks.
-template<int NS, bool JAC>
+// jac = false (uniform) leaves J alone.  With WD, also the destruction rates.
+// Stoichiometry is walked through each reaction's species lists (a few entries) rather than all species, the net rate
+// of a reaction added once per species; the Jacobian keeps static indices (register-resident) and skips rows and
+// columns through the reaction's species bit masks.
+template<int NS, bool JAC, bool WD = false>
 __device__ __forceinline__ void source(const ChemMech &m, double t, const double *rhoY, double *w, double *J,
-                                       double *wd = nullptr, double floor = 1e-30) {
-  double c[NS], g[NS], cr[NS], de[NS];
+                                       double *wd = nullptr, double floor = 1e-30, bool jac = JAC) {
+  double c[NS], g[NS], net[NS], de[NS];
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
     c[l] = rhoY[l] * m.imw[l] * 1e-3;
-    cr[l] = 0;
+    net[l] = 0;
     de[l] = 0;
   }
   if constexpr (JAC) {
+    if (jac)
 #pragma unroll
-    for (int q = 0; q < NS * NS; ++q) J[q] = 0;
+      for (int q = 0; q < NS * NS; ++q) J[q] = 0;
   }
   // Equilibrium constants are needed unless every reversible reaction carries explicit REV parameters
   // (FiniteRateChem.cu:1519-1557); then they are applied to every reaction of type other than 0 and 2.
   const double lnT = log(t), iT = 1.0 / t;
   if (m.need_gibbs) gibbs<NS>(m, t, lnT, iT, g);
-  const double tp = kPatm / kRu * 1e-3 / t;
+  // p_atm / (R T) in kmol/m^3 and its reciprocal
+  const double tp = kPatm / kRu * 1e-3 * iT, itp = kRu / kPatm * 1e+3 * t;
   for (int r = 0; r < m.nr; ++r) {
-    const int ty = m.type[r];
-    const int nfs = m.nfs[r], nbs = m.nbs[r];
-    double kf = arrhenius(lnT, iT, m.A[r], m.b[r], m.Ea[r]);
+    const ReacRecord q = m.rec[r];
+    const int ty = q.type;
+    const int nfs = q.n_sides & 255, nbs = q.n_sides >> 8;
+    auto sp = [](unsigned s, int k) { return (int)(s >> 8 * k & 255u); };
+    auto nu = [](unsigned long long s, int k) { return (int)(short)(s >> 16 * k & 65535u); };
+    double kf = arrhenius(lnT, iT, q.A, q.b, q.Ea);
     double cc = 0;
     if (ty >= 4) {
+      double tb[NS];
 #pragma unroll
-      for (int l = 0; l < NS; ++l) cc += c[l] * m.tb[r][l];
+      for (int l = 0; l < NS; ++l) tb[l] = m.tb[r][l];
+#pragma unroll
+      for (int l = 0; l < NS; ++l) cc += c[l] * tb[l];
     }
     if (ty == 3) {
-      kf += arrhenius(lnT, iT, m.A2[r], m.b2[r], m.Ea2[r]);
+      kf += arrhenius(lnT, iT, q.A2, q.b2, q.Ea2);
     } else if (ty == 4) {
       kf *= cc;
     } else if (ty > 4) {
-      const double klow = arrhenius(lnT, iT, m.A2[r], m.b2[r], m.Ea2[r]), khigh = kf;
+      const double klow = arrhenius(lnT, iT, q.A2, q.b2, q.Ea2), khigh = kf;
       if (khigh < 1e-25 && klow < 1e-25) {
         kf = 0;
       } else {
         const double pr = klow * cc / khigh;
         double F = 1.0;
         if (ty > 5) {
-          double fc = (1 - m.troe[r][0]) * exp(-t / m.troe[r][1]) + m.troe[r][0] * exp(-t / m.troe[r][2]);
-          if (ty == 7) fc += exp(-m.troe[r][3] / t);
+          double fc = (1 - q.troe[0]) * exp(-t / q.troe[1]) + q.troe[0] * exp(-t / q.troe[2]);
+          if (ty == 7) fc += exp(-q.troe[3] * iT);
           const double lfc = log10(fc);
           const double cq = -0.4 - 0.67 * lfc, nq = 0.75 - 1.27 * lfc;
           const double lpr = log10(pr);
@@ -132,55 +178,62 @@ __device__ __forceinline__ void source(const ChemMech &m, double t, const double
       }
     }
     double kb = 0;
-    if (ty != 0 && m.rev[r] == 1) {
-      kb = arrhenius(lnT, iT, m.A2[r], m.b2[r], m.Ea2[r]);
+    if (ty != 0 && q.rev == 1) {
+      kb = arrhenius(lnT, iT, q.A2, q.b2, q.Ea2);
       if (ty == 4) kb *= cc;
     }
     if (m.need_gibbs && ty != 0 && ty != 2) {
       double dg = 0;
-      for (int s = 0; s < nbs; ++s) dg += g[m.bsp[r][s]] * m.bnu[r][s];
-      for (int s = 0; s < nfs; ++s) dg -= g[m.fsp[r][s]] * m.fnu[r][s];
-      kb = kf / (int_pow(tp, m.iorder[r]) * exp(-dg));
+      for (int s = 0; s < nbs; ++s) dg += g[sp(q.bsp, s)] * nu(q.bnu, s);
+      for (int s = 0; s < nfs; ++s) dg -= g[sp(q.fsp, s)] * nu(q.fnu, s);
+      // kf / ((p_atm / R T)^order exp(-dg)), without dividing
+      kb = kf * exp(dg) * int_pow(q.iorder < 0 ? tp : itp, q.iorder < 0 ? -q.iorder : q.iorder);
     }
     double q1 = 1.0, q2 = ty != 0 ? 1.0 : 0.0;
-    for (int s = 0; s < nfs; ++s) q1 *= int_pow(c[m.fsp[r][s]], m.fnu[r][s]);
+    for (int s = 0; s < nfs; ++s) q1 *= int_pow(c[sp(q.fsp, s)], nu(q.fnu, s));
     if (ty != 0)
-      for (int s = 0; s < nbs; ++s) q2 *= int_pow(c[m.bsp[r][s]], m.bnu[r][s]);
+      for (int s = 0; s < nbs; ++s) q2 *= int_pow(c[sp(q.bsp, s)], nu(q.bnu, s));
     q1 *= kf;
     q2 *= kb;
+    const double qn = q1 - q2;
     for (int s = 0; s < nfs; ++s) {
-      const int l = m.fsp[r][s];
-      const double nu = m.fnu[r][s];
-      cr[l] += q2 * nu;
-      de[l] += q1 * nu;
+      const int l = sp(q.fsp, s);
+      const double n = nu(q.fnu, s);
+      net[l] -= qn * n;
+      if constexpr (WD) de[l] += q1 * n;
     }
     for (int s = 0; s < nbs; ++s) {
-      const int l = m.bsp[r][s];
-      const double nu = m.bnu[r][s];
-      cr[l] += q1 * nu;
-      de[l] += q2 * nu;
+      const int l = sp(q.bsp, s);
+      const double n = nu(q.bnu, s);
+      net[l] += qn * n;
+      if constexpr (WD) de[l] += q2 * n;
     }
     if constexpr (JAC) {
-      const unsigned um = m.umask[r], am = m.amask[r];
-      double v[NS];
+      if (!jac) continue;
+      // the rows of the stoichiometric tables whole, a few wide loads, instead of entry by entry behind the mask bits
+      const unsigned um = q.umask, am = q.amask;
+      double v[NS], dn[NS];
 #pragma unroll
-      for (int n = 0; n < NS; ++n) v[n] = (um >> n & 1u) ? m.nf[r][n] * q1 - m.nb[r][n] * q2 : 0.0;
+      for (int n = 0; n < NS; ++n) {
+        v[n] = m.nf[r][n] * q1 - m.nb[r][n] * q2;
+        dn[n] = m.dnu[r][n];
+      }
 #pragma unroll
       for (int a = 0; a < NS; ++a) {
         if (!(am >> a & 1u)) continue;
-        const double dn = m.dnu[r][a];
 #pragma unroll
         for (int n = 0; n < NS; ++n)
-          if (um >> n & 1u) J[a * NS + n] += dn * v[n];
+          if (um >> n & 1u) J[a * NS + n] += dn[a] * v[n];
       }
     }
   }
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
-    w[l] = cr[l] * (1e+3 * m.mw[l]) - de[l] * (1e+3 * m.mw[l]);
-    if (wd) wd[l] = de[l] * (1e+3 * m.mw[l]);
+    w[l] = net[l] * (1e+3 * m.mw[l]);
+    if constexpr (WD) wd[l] = de[l] * (1e+3 * m.mw[l]);
   }
   if constexpr (JAC) {
+    if (!jac) return;
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
       const double inv = rhoY[n] > floor ? 1.0 / rhoY[n] : 0.0;
@@ -213,7 +266,8 @@ template<int NS> __device__ __forceinline__ void lu(double *a, int *piv) {
     piv[k] = ik;
     // row exchange through value selects: every index stays static and no branch is formed (a branch per
     // candidate row lets the optimiser merge them into stores through a chosen address, which sends the
-    // whole matrix to scratch memory)
+    // whole matrix to scratch memory); skipped where no lane exchanges anything, as in all but the stiff cells
+    if (__any(ik != k))
 #pragma unroll
     for (int r = k + 1; r < NS; ++r) {
       const bool sw = r == ik;
@@ -238,6 +292,7 @@ template<int NS> __device__ __forceinline__ void lu(double *a, int *piv) {
 template<int NS> __device__ __forceinline__ void lu_solve(const double *a, const int *piv, double *b) {
 #pragma unroll
   for (int r = 0; r < NS; ++r) {
+    if (__any(piv[r] != r))
 #pragma unroll
     for (int q = r + 1; q < NS; ++q) {
       const bool sw = piv[r] == q;
@@ -259,29 +314,67 @@ template<int NS> __device__ __forceinline__ void lu_solve(const double *a, const
   }
 }
 
-// Newton iteration for T at fixed specific internal energy E (ConstVolumeReactor.cpp:970-995).
-template<int NS> __device__ double update_t(const ChemMech &m, double t, const double *yk, double E) {
-  double imw = 0;
-#pragma unroll
-  for (int l = 0; l < NS; ++l) imw += yk[l] * m.imw[l];
-  const double R = kRu * imw;
+// Newton iteration T -> T - (h - R T - e) / (cp - R) for the mixture of mass fractions yk until the relative change is
+// at most tol (at most `most` times).  With a common fit range the iteration runs on the mixture's own fit (54 products,
+// again for a lane that crosses the middle of the range) instead of nine species fits per iteration.
+template<int NS>
+__device__ __forceinline__ double newton_t(const ChemMech &m, double t, const double *yk, double R, double E, double tol, int most) {
   double err = 1e+6;
-  for (int it = 0; it < 100 && err > 1e-8; ++it) {
-    // h_cp species by species, summed as they come (the same operations in the same order as summing the
-    // arrays h_cp fills, without holding them)
-    double cpt = 0, hh = 0;
+  int it = 0;
+  if (m.common_range) {
+    double C[6];
+    int side = -1; // 0: C holds the low fit, 1: the high one
+#pragma unroll 1
+    for (; it < most && err > tol; ++it) {
+      const int now = t < m.ct_mid ? 0 : 1;
+      if (__any(now != side)) {
+        const bool fresh = now != side;
+        auto mix = [&](const double(*c)[7]) {
+          double D[6] = {};
+#pragma unroll
+          for (int l = 0; l < NS; ++l) {
+            const double yr = yk[l] * (kRu * m.imw[l]);
+#pragma unroll
+            for (int q = 0; q < 6; ++q) D[q] = fma(yr, c[l][q], D[q]);
+          }
+#pragma unroll
+          for (int q = 0; q < 6; ++q) C[q] = fresh ? D[q] : C[q];
+        };
+        if (__all(now == 0)) mix(m.lo);
+        else if (__all(now == 1)) mix(m.hi);
+        else mix(now ? m.hi : m.lo);
+        side = now;
+      }
+      double h, cp;
+      h_cp_fit(C, 1.0, t, fmin(fmax(t, m.ct_low), m.ct_high), h, cp);
+      const double t1 = t - (h - R * t - E) / (cp - R);
+      err = fabs(1 - t1 / t);
+      t = t1;
+    }
+    return t;
+  }
+#pragma unroll 1
+  for (; it < most && err > tol; ++it) {
+    double h[NS], cp[NS], cpt = 0, hh = 0;
+    h_cp<NS>(m, t, h, cp);
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      double h1, cp1;
-      h_cp_one(m, l, t, h1, cp1);
-      cpt += cp1 * yk[l];
-      hh += h1 * yk[l];
+      cpt += cp[l] * yk[l];
+      hh += h[l] * yk[l];
     }
     const double t1 = t - (hh - R * t - E) / (cpt - R);
     err = fabs(1 - t1 / t);
     t = t1;
   }
   return t;
+}
+
+// T at fixed specific internal energy E (ConstVolumeReactor.cpp:970-995).
+template<int NS> __device__ __forceinline__ double update_t(const ChemMech &m, double t, const double *yk, double E) {
+  double imw = 0;
+#pragma unroll
+  for (int l = 0; l < NS; ++l) imw += yk[l] * m.imw[l];
+  return newton_t<NS>(m, t, yk, kRu * imw, E, 1e-8, 100);
 }
 
 // Collision integral of binary diffusion at reduced temperature t (Transport.cu:188-190),

@@ -332,7 +332,40 @@ ChemMech parse_mechanism(const std::string &mech_text, const std::string &therm_
     }
     m.iorder[r] = (int)m.order[r];
     if ((double)m.iorder[r] != m.order[r]) throw std::runtime_error("non-integer reaction order");
+    ReacRecord &q = m.rec[r];
+    q = {m.A[r], m.b[r], m.Ea[r], m.A2[r], m.b2[r], m.Ea2[r], {m.troe[r][0], m.troe[r][1], m.troe[r][2], m.troe[r][3]},
+         m.type[r], m.rev[r], m.iorder[r], m.nfs[r] | m.nbs[r] << 8, 0, 0, 0, 0, m.umask[r], m.amask[r]};
+    auto pack = [](int n, const int *sp, const int *nu, unsigned &s, unsigned long long &c) {
+      for (int k = 0; k < n; ++k) {
+        if (nu[k] < -32767 || nu[k] > 32767) throw std::runtime_error("stoichiometric coefficient out of range");
+        s |= (unsigned)sp[k] << 8 * k;
+        c |= (unsigned long long)(unsigned short)(short)nu[k] << 16 * k;
+      }
+    };
+    pack(m.nfs[r], m.fsp[r], m.fnu[r], q.fsp, q.fnu);
+    pack(m.nbs[r], m.bsp[r], m.bnu[r], q.bsp, q.bnu);
   }
+  m.max_f = m.max_b = 0;
+  int at = 0;
+  for (int falloff = 0; falloff < 2; ++falloff)
+    for (int r = 0; r < nr; ++r)
+      if ((m.type[r] > 4) == (falloff == 1)) m.by_cost[at++] = r;
+  for (int r = 0; r < nr; ++r) {
+    m.max_f = std::max(m.max_f, m.nfs[r]);
+    m.max_b = std::max(m.max_b, m.nbs[r]);
+  }
+  m.common_range = 1;
+  for (int k = 1; k < m.ns; ++k)
+    if (m.t_low[k] != m.t_low[0] || m.t_mid[k] != m.t_mid[0] || m.t_high[k] != m.t_high[0]) m.common_range = 0;
+  m.ct_low = m.t_low[0];
+  m.ct_mid = m.t_mid[0];
+  m.ct_high = m.t_high[0];
+  m.c_ln_low = m.ln_t_low[0];
+  m.c_ln_high = m.ln_t_high[0];
+  m.c_inv_low = m.inv_t_low[0];
+  m.c_inv_high = m.inv_t_high[0];
+  // a range out of order has no "side of the middle"
+  if (!(m.ct_low <= m.ct_mid && m.ct_mid <= m.ct_high)) m.common_range = 0;
   return m;
 }
 

@@ -729,21 +729,7 @@ __device__ __forceinline__ double mix_state(const ChemMech &m, double *q, double
   }
   // Newton iteration for T at fixed e, |1 - T1/T| < 1e-5, at most 1000 iterations
   const double e = q[4] * di - 0.5 * (u * u + v * v + w * w);
-  double t = t0, err = 1;
-  for (int it = 0; it < 1000 && err > 1e-5; ++it) {
-    double h[NS], cp[NS];
-    chemdev::h_cp<NS>(m, t, h, cp);
-    double cpt = 0, hh = 0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      cpt += cp[l] * y[l];
-      hh += h[l] * y[l];
-    }
-    const double t1 = t - (hh - R * t - e) / (cpt - R);
-    err = fabs(1 - t1 / t);
-    t = t1;
-  }
-  return t;
+  return chemdev::newton_t<NS>(m, t0, y, R, e, 1e-5, 1000);
 }
 
 // cn: the frozen transport residual of Wu's splitting (update_cv_and_bv_rk_wu, StrangSplitting.cu:504-562:
@@ -788,7 +774,7 @@ __global__ __launch_bounds__(256) void k_mix_update(DevBlock b, MixArrays x, int
     double ry[NS], w[NS], wd[NS];
 #pragma unroll
     for (int l = 0; l < NS; ++l) ry[l] = rho * x.sv[id + l * sz];
-    chemdev::source<NS, false>(*x.mech, b.bv[id + 5 * sz], ry, w, nullptr, wd);
+    chemdev::source<NS, false, true>(*x.mech, b.bv[id + 5 * sz], ry, w, nullptr, wd);
     const double J = b.jac[id];
     double ts = 1e+6;
 #pragma unroll
@@ -1285,7 +1271,7 @@ __global__ __launch_bounds__(256) void k_mix_wu_reaction(DevBlock b, MixArrays x
     if constexpr (METHOD == 1) {
       double a[NS * NS];
       int piv[NS];
-      chemdev::source<NS, true>(m, t, q + 5, w, a, wd, 1e-25);
+      chemdev::source<NS, true, true>(m, t, q + 5, w, a, wd, 1e-25);
 #pragma unroll
       for (int r = 0; r < NS; ++r)
 #pragma unroll
@@ -1293,7 +1279,7 @@ __global__ __launch_bounds__(256) void k_mix_wu_reaction(DevBlock b, MixArrays x
       chemdev::lu<NS>(a, piv);
       chemdev::lu_solve<NS>(a, piv, w);
     } else {
-      chemdev::source<NS, false>(m, t, q + 5, w, nullptr, wd);
+      chemdev::source<NS, false, true>(m, t, q + 5, w, nullptr, wd);
     }
     if constexpr (METHOD == 3) {
       double qn[NV];

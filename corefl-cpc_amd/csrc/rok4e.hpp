@@ -13,8 +13,18 @@ constexpr double G41 = 0.992356412977094 / G, G42 = -1.390032613873701 / G, G43 
 constexpr double B1 = 0.194335256262729, B2 = 0.483167813989227, B4 = 0.322496929748044;
 constexpr double E1 = -0.217819895945721 - B1, E2 = 1.03130847478467 - B2, E3 = 0.186511421161047, E4 = -B4;
 
+// By stage: the weights of k1, k2 in the stage's state, and of k1, k2, k3 in its right-hand side.
+__constant__ const double kStageA[4][2] = {{0, 0}, {A21, 0}, {A31, A32}, {A31, A32}};
+__constant__ const double kStageG[4][3] = {{0, 0, 0}, {G21, 0, 0}, {G31, G32, 0}, {G41, G42, G43}};
+
 // A step whose size h satisfies kStretch h >= (time left in the interval) is taken to the interval's end.
 constexpr double kStretch = 1.05;
+
+// The PI controller's step factor after the first step, 0.8 err_last^0.1 (err + 1e-20)^-0.175 in [0.2, 5], its two powers
+// as one exponential of logarithms.
+__device__ __forceinline__ double step_factor(double err_last, double err) {
+  return fmin(5.0, fmax(0.2, 0.8 * exp(0.1 * log(err_last) - 0.175 * log(err + 1e-20))));
+}
 
 } // namespace rok4e
 } // namespace corefl

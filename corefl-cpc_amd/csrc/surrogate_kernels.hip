@@ -460,7 +460,7 @@ struct ThermoLds {
   double t_low[9], t_mid[9], t_high[9], R[9], imw[9];
 };
 
-// h and cp of species i at t from the LDS table: chemdev::h_cp_one's operations in its order.
+// h and cp of species i at t from the LDS table: the fit inside its range, continued linearly outside.
 __device__ __forceinline__ void h_cp_lds(const ThermoLds &th, int i, double t, double &h, double &cp) {
   using chemdev::kThird;
   const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t5 = t4 * t;
