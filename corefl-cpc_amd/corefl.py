@@ -447,7 +447,7 @@ class Chemistry:
 
     def set_launch(self, mode, threads=64, blocks=1024, budget=0):
         """mode 0: one thread per cell; 1: work queue; 2: cooperative (16 lanes per cell); 3: work queue for
-        `budget` attempts, then cooperative.  A bool mode means 1 (True) or 0 (False)."""
+        at least `budget` attempts, then cooperative for the last cells.  A bool mode means 1 (True) or 0 (False)."""
         _check(self._lib.corefl_chem_set_launch(self._ctx, int(mode), int(threads), int(blocks), int(budget)))
 
     def get_launch(self):

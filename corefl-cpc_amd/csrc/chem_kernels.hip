@@ -31,64 +31,80 @@ template<int NS> struct Cell {
   int steps, rejects, attempts;
 };
 
-// One ROK4E attempt (ConstVolumeReactor.cpp:173-476 with adaptive_time_step = 1).
+// One ROK4E attempt (ConstVolumeReactor.cpp:173-476 with adaptive_time_step = 1): four stages over the third stage's
+// source, and a last pass for the new temperature.  The stages are one loop around a single copy of the source, the
+// temperature iteration and the solve: written out, the kernel is 113 KB of code, more than the 64 KB instruction cache
+// of two CUs; rolled it is 57 KB.  An attempt of a wave takes 100 us, from 145 (2.1M igniting cells: 3.4 ms, from 4.9):
+// 21700 vector instructions (28600), 670 scalar loads (2060) and no vector loads of coefficients.  It is bound by its one
+// wave per SIMD: vector instructions are 37% of its cycles, scalar ones 24%, waits for scalar loads 27%.  Two waves at 256
+// registers keep 950 bytes a lane in scratch and take 4.9 ms.
 template<int NS>
-__device__ __forceinline__ void rok4e_attempt(const ChemMech &m, Cell<NS> &s, double rtol, double atol) {
+__device__ __forceinline__ void rok4e_attempt(const ChemMech *mp, Cell<NS> &s, double rtol, double atol) {
   const double dt = s.dt;
-  double w[NS], J[NS * NS], k1[NS], k2[NS], k3[NS], k4[NS], ys[NS], yk[NS];
+  double w[NS], J[NS * NS], k1[NS], k2[NS], k3[NS], ys[NS];
   int piv[NS];
-  source<NS, true>(m, s.T, s.y, w, J);
   // The step ends the interval when it would leave less than 5% of itself (no sliver step, whose size
   // would otherwise become the proposal carried to the next sub-step).
   const double rem = dt - s.time;
   const double hs = s.h * kStretch >= rem ? rem : s.h;
-#pragma unroll
-  for (int q = 0; q < NS * NS; ++q) J[q] = -hs * G * J[q];
-#pragma unroll
-  for (int l = 0; l < NS; ++l) J[l * NS + l] += 1.0;
-  lu<NS>(J, piv);
-#pragma unroll
-  for (int l = 0; l < NS; ++l) k1[l] = w[l];
-  lu_solve<NS>(J, piv, k1);
   const double irho = 1.0 / s.rho; // products by 1/rho stand for the reference's divisions
 #pragma unroll
-  for (int l = 0; l < NS; ++l) {
-    ys[l] = s.y[l] + hs * A21 * k1[l];
-    yk[l] = ys[l] * irho;
+  for (int l = 0; l < NS; ++l) k1[l] = k2[l] = k3[l] = 0;
+  double Ts = s.T, err = 0;
+#pragma unroll 1
+  for (int st = 0; st < 5; ++st) {
+    const ChemMech &m = opaque(mp);
+    if (st != 3) { // the fourth stage takes the third's source
+      if (st < 4) {
+        const double a1 = hs * kStageA[st][0], a2 = hs * kStageA[st][1];
+#pragma unroll
+        for (int l = 0; l < NS; ++l) ys[l] = s.y[l] + (a1 * k1[l] + a2 * k2[l]);
+      }
+      // st 4: ys is the new state, and an accepted step gets its temperature from the old one
+      if (st > 0 && (st < 4 || err <= 1)) {
+        double yk[NS];
+#pragma unroll
+        for (int l = 0; l < NS; ++l) yk[l] = ys[l] * irho;
+        Ts = update_t<NS>(m, st == 4 ? s.T : Ts, yk, s.E);
+      }
+      if (st == 4) break;
+      source<NS, true>(m, Ts, ys, w, J, nullptr, 1e-30, st == 0);
+      if (st == 0) {
+#pragma unroll
+        for (int q = 0; q < NS * NS; ++q) J[q] = -hs * G * J[q];
+#pragma unroll
+        for (int l = 0; l < NS; ++l) J[l * NS + l] += 1.0;
+        lu<NS>(J, piv);
+      }
+    }
+    const double g1 = kStageG[st][0], g2 = kStageG[st][1], g3 = kStageG[st][2];
+    double k[NS];
+#pragma unroll
+    for (int l = 0; l < NS; ++l) k[l] = w[l] + (g1 * k1[l] + g2 * k2[l] + g3 * k3[l]);
+    lu_solve<NS>(J, piv, k);
+#pragma unroll
+    for (int l = 0; l < NS; ++l) k[l] -= g1 * k1[l] + g2 * k2[l] + g3 * k3[l];
+    if (st == 0) {
+#pragma unroll
+      for (int l = 0; l < NS; ++l) k1[l] = k[l];
+    } else if (st == 1) {
+#pragma unroll
+      for (int l = 0; l < NS; ++l) k2[l] = k[l];
+    } else if (st == 2) {
+#pragma unroll
+      for (int l = 0; l < NS; ++l) k3[l] = k[l];
+    } else {
+#pragma unroll
+      for (int l = 0; l < NS; ++l) {
+        ys[l] = s.y[l] + hs * (B1 * k1[l] + B2 * k2[l] + B4 * k[l]);
+        const double dy = hs * (E1 * k1[l] + E2 * k2[l] + E3 * k3[l] + E4 * k[l]) / (rtol * ys[l] + atol);
+        err += dy * dy;
+      }
+      err = sqrt(err / NS);
+    }
   }
-  double Ts = update_t<NS>(m, s.T, yk, s.E);
-  source<NS, false>(m, Ts, ys, w, nullptr);
-#pragma unroll
-  for (int l = 0; l < NS; ++l) k2[l] = w[l] + G21 * k1[l];
-  lu_solve<NS>(J, piv, k2);
-#pragma unroll
-  for (int l = 0; l < NS; ++l) {
-    k2[l] -= G21 * k1[l];
-    ys[l] = s.y[l] + hs * (A31 * k1[l] + A32 * k2[l]);
-    yk[l] = ys[l] * irho;
-  }
-  Ts = update_t<NS>(m, Ts, yk, s.E);
-  source<NS, false>(m, Ts, ys, w, nullptr);
-#pragma unroll
-  for (int l = 0; l < NS; ++l) k3[l] = w[l] + G31 * k1[l] + G32 * k2[l];
-  lu_solve<NS>(J, piv, k3);
-#pragma unroll
-  for (int l = 0; l < NS; ++l) {
-    k3[l] -= G31 * k1[l] + G32 * k2[l];
-    k4[l] = w[l] + G41 * k1[l] + G42 * k2[l] + G43 * k3[l];
-  }
-  lu_solve<NS>(J, piv, k4);
-  double err = 0, ynew[NS];
-#pragma unroll
-  for (int l = 0; l < NS; ++l) {
-    k4[l] -= G41 * k1[l] + G42 * k2[l] + G43 * k3[l];
-    ynew[l] = s.y[l] + hs * (B1 * k1[l] + B2 * k2[l] + B4 * k4[l]);
-    const double dy = hs * (E1 * k1[l] + E2 * k2[l] + E3 * k3[l] + E4 * k4[l]) / (rtol * ynew[l] + atol);
-    err += dy * dy;
-  }
-  err = sqrt(err / NS);
   double hstar = hs;
-  if (s.steps > 0) hstar *= fmin(5.0, fmax(0.2, 0.8 * pow(s.err_last, 0.1) * pow(err + 1e-20, -0.175)));
+  if (s.steps > 0) hstar *= step_factor(s.err_last, err);
   else if (!(err <= 1)) hstar *= 0.2; // a NaN first-step error also cuts the step (the reference would repeat it)
   // a step cut short by the end of the interval does not shrink the proposal
   if (err <= 1 && hs < s.h) hstar = fmax(hstar, s.h);
@@ -96,13 +112,10 @@ __device__ __forceinline__ void rok4e_attempt(const ChemMech &m, Cell<NS> &s, do
   ++s.attempts;
   if (err <= 1) {
 #pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      s.y[l] = ynew[l];
-      yk[l] = ynew[l] * irho;
-    }
+    for (int l = 0; l < NS; ++l) s.y[l] = ys[l];
     s.time += hs;
     s.err_last = fmax(err, 1e-30); // an exactly zero error would stall the PI controller (0^0.1 = 0)
-    s.T = update_t<NS>(m, s.T, yk, s.E);
+    s.T = Ts;
     ++s.steps;
   } else {
     ++s.rejects;
@@ -142,10 +155,9 @@ __global__ __launch_bounds__(256) void k_chem_static(const ChemMech *__restrict_
   const int w = blockIdx.x * blockDim.x + threadIdx.x;
   if (w >= work_count(b)) return;
   const int c = work_cell(b, w);
-  const ChemMech &m = *mp;
   Cell<NS> s;
   load_cell<NS>(b, c, dt, s);
-  while (s.time < s.dt && s.attempts < max_attempts) rok4e_attempt<NS>(m, s, rtol, atol);
+  while (s.time < s.dt && s.attempts < max_attempts) rok4e_attempt<NS>(mp, s, rtol, atol);
   store_cell<NS>(b, c, s, s.time >= s.dt);
 }
 
@@ -161,13 +173,15 @@ template<int NS> __device__ __forceinline__ void store_partial(const ChemBatch &
   b.elast[c] = s.err_last;
 }
 
-// budget > 0: a cell still unfinished after `budget` attempts is handed over (appended to b.defer) instead
-// of holding its lane for the rest of its chain.
+// budget > 0: a cell still unfinished after `budget` attempts is handed over (appended to b.defer) once fewer than 3/16
+// of the launch's lanes hold a cell.  An attempt of every cell takes 100 us here whatever their number up to one per
+// lane (65536 lanes), and in the cooperative kernel 60 us for every 8192 cells, so the lines cross near 13000 cells;
+// below, its shorter attempt counts.  (200003 igniting cells, 5.6 attempts on average and 123 at most: 5.8 ms, 6.7 with
+// every cell handed over after its fourth attempt.)
 template<int NS>
 __global__ __launch_bounds__(256) void k_chem_queue(const ChemMech *__restrict__ mp, ChemBatch b, double dt,
                                                     double rtol, double atol, int max_attempts, int *counter,
                                                     int budget) {
-  const ChemMech &m = *mp;
   const int lane = __lane_id();
   const int n_work = work_count(b);
   Cell<NS> s;
@@ -194,7 +208,7 @@ __global__ __launch_bounds__(256) void k_chem_queue(const ChemMech *__restrict__
     if (__ballot(cell >= 0) == 0) break;
     bool defer = false;
     if (cell >= 0) {
-      rok4e_attempt<NS>(m, s, rtol, atol);
+      rok4e_attempt<NS>(mp, s, rtol, atol);
       if (s.time >= s.dt || s.attempts >= max_attempts) {
         store_cell<NS>(b, cell, s, s.time >= s.dt);
         cell = -1;
@@ -202,7 +216,15 @@ __global__ __launch_bounds__(256) void k_chem_queue(const ChemMech *__restrict__
         defer = budget > 0 && s.attempts >= budget;
       }
     }
-    const unsigned long long dm = __ballot(defer);
+    unsigned long long dm = __ballot(defer);
+    if (dm) {
+      // every lane that found the queue empty has counted once more, so the lanes at work are the others
+      int fetched = 0;
+      if (lane == 0) fetched = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const long lanes = (long)gridDim.x * blockDim.x, idle = (long)__shfl(fetched, 0, 64) - n_work;
+      if (idle < 0 || 16 * (lanes - idle) > 3 * lanes) defer = false;
+      dm = __ballot(defer);
+    }
     if (dm) {
       const int leader = __ffsll((long long)dm) - 1;
       int base = 0;

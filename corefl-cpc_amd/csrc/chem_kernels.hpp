@@ -39,8 +39,8 @@ __device__ __forceinline__ double cell_dt(const ChemBatch &b, long c, double dt)
 // Launch shape picked by the autotuner.
 struct ChemLaunch {
   int queue;   // 0: one lane per cell; 1: persistent work queue, one lane per cell; 2: persistent work queue,
-               // 16 lanes per cell (cooperative); 3: mode 1 for at most `budget` attempts per cell, the
-               // unfinished cells then continued by mode 2
+               // 16 lanes per cell (cooperative); 3: mode 1 for at least `budget` attempts per cell, the
+               // cells unfinished when few are left then continued by mode 2
   int threads; // workgroup size (multiple of 64)
   int blocks;  // persistent workgroups (modes 1-3)
   int budget;  // attempt budget of mode 3

@@ -243,8 +243,8 @@ int corefl_chem_integrate(corefl_chem *chem, double dt, double rtol, double atol
 /* Launch shape of corefl_chem_integrate (no reference counterpart: the reference integrates one cell per
  * thread, src/FiniteRateChem.cu:1388).  mode 0: one thread per cell; 1: persistent waves fetching cells
  * from a device counter, `blocks` workgroups; 2: persistent waves integrating four cells at a time, 16 lanes
- * per cell (lower latency per step attempt, for stiff cells); 3: mode 1 for at most `budget` attempts per
- * cell, the unfinished cells then continued by mode 2.  All modes give the same result to rounding.
+ * per cell (lower latency per step attempt, for stiff cells); 3: mode 1 for at least `budget` attempts per
+ * cell, the cells unfinished when few are left then continued by mode 2.  All modes give the same result to rounding.
  * threads is 64, 128 or 256; budget is used by mode 3 only. */
 int corefl_chem_set_launch(corefl_chem *chem, int mode, int threads, int blocks, int budget);
 int corefl_chem_get_launch(const corefl_chem *chem, int *mode, int *threads, int *blocks, int *budget);
