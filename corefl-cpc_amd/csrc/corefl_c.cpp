@@ -469,7 +469,7 @@ struct corefl_ctx {
     for (auto &b : blocks) {
       if (ns) {
         if (scheme.inviscid_scheme == 2) HIPCHK(corefl::launch_mix_entropy_fix(b.dev, b.mix, scheme, s));
-        for (int d = 0; d < b.dev.dim; ++d) HIPCHK(corefl::launch_mix_inviscid_flux(b.dev, b.mix, scheme, d, s));
+        HIPCHK(corefl::launch_mix_inviscid_flux(b.dev, b.mix, scheme, s));
       } else {
         if (scheme.inviscid_scheme == 2) HIPCHK(corefl::launch_entropy_fix(b.dev, scheme, s));
         HIPCHK(corefl::launch_inviscid_flux(b.dev, scheme, 7u, s));

@@ -37,8 +37,8 @@ hipError_t launch_mix_inner_exchange(const DevBlock &b, const MixArrays &x, cons
                                      const DevInner &f, hipStream_t s);
 hipError_t launch_mix_entropy_fix(const DevBlock &b, const MixArrays &x, const Scheme &sc, hipStream_t s);
 // reconstruction 1 first order, 2 MUSCL, 3 NND2 (minmod), 4 / 5 component-wise WENO5 / WENO7;
-// inviscid_scheme 2 Roe, 3 AUSM+, 4 HLLC.
-hipError_t launch_mix_inviscid_flux(const DevBlock &b, const MixArrays &x, const Scheme &sc, int dir, hipStream_t s);
+// inviscid_scheme 2 Roe, 3 AUSM+, 4 HLLC.  All directions of the block in one launch.
+hipError_t launch_mix_inviscid_flux(const DevBlock &b, const MixArrays &x, const Scheme &sc, hipStream_t s);
 hipError_t launch_mix_update(const DevBlock &b, const MixArrays &x, int rk, const double *dt_dev, bool rhs_only,
                              hipStream_t s);
 // Wu's splitting (temporal_scheme 4): the reaction sub-step with the frozen transport residual held in b.dq,
