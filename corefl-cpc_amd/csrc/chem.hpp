@@ -19,6 +19,9 @@ struct ReacRecord {
 };
 static_assert(sizeof(ReacRecord) == 128, "one reaction in two 64-byte scalar loads");
 
+constexpr int kOmegaOctaves = 40, kOmegaTable = 16 * kOmegaOctaves;
+constexpr double kOmegaShift = 0.55909, kOmegaPower = 2.1705, kOmegaSlow = 0.15504;
+
 // Plain data, copied to device memory once and read uniformly by every lane.
 struct ChemMech {
   int ns, nr, ne;
@@ -65,9 +68,16 @@ struct ChemMech {
   int geometry[kMaxSpec];
   double lj_inv[kMaxSpec], vis_coeff[kMaxSpec], zrot[kMaxSpec];
   double wdw[kMaxSpec][kMaxSpec], sqw[kMaxSpec][kMaxSpec], bdc[kMaxSpec][kMaxSpec], kbe[kMaxSpec][kMaxSpec];
-  // ln(1 / (eps / k_B)), ln(k_B / eps_jk) and 1 / bdc: the logarithms turn the collision integrals' powers of
-  // T* = T k_B / eps into exponentials of ln T + ln(k_B / eps), with one ln T per node
-  double log_lj_inv[kMaxSpec], log_kbe[kMaxSpec][kMaxSpec], inv_bdc[kMaxSpec][kMaxSpec];
+  // ln(1 / (eps / k_B)), which turns the viscosities' powers of T* = T k_B / eps into exponentials of
+  // ln T + ln(k_B / eps) with one ln T per node, and 1 / bdc
+  double log_lj_inv[kMaxSpec], inv_bdc[kMaxSpec][kMaxSpec];
+  // The collision integral of binary diffusion, 1.0548 T*^-0.15504 + (T* + 0.55909)^-2.1705: the first term's part
+  // that no temperature changes, 1.0548 (k_B / eps_jk)^-0.15504, as the unevaluated sum omega_hi + omega_lo; for the
+  // second a table over the sixteenths of the octaves from 1/2 up, {s, s^2.1705} with s near the reciprocal of the
+  // sixteenth's middle, so that x^-2.1705 = s^2.1705 (x s)^-2.1705 is a short series about 1.  t_omega: the temperature
+  // up to which every T* + 0.55909 lies in the table (over 10^12 K; the second term is below an ulp of the first there).
+  double omega_hi[kMaxSpec][kMaxSpec], omega_lo[kMaxSpec][kMaxSpec], t_omega;
+  double omega_table[kOmegaTable][2];
 };
 
 // h_k and cp_k per unit mass at t, linear extrapolation outside [t_low, t_high] (Thermo.cu:470-520).

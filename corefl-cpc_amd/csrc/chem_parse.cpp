@@ -428,11 +428,31 @@ void parse_transport(const std::string &tran_text, ChemMech &m) {
       m.kbe[j][k] = m.kbe[k][j] = 1.0 / (xi * xi * std::sqrt(eps[j] * eps[k]));
     }
   }
+  double kbe_max = 0;
   for (int j = 0; j < ns; ++j) {
     m.log_lj_inv[j] = std::log(m.lj_inv[j]);
     for (int k = 0; k < ns; ++k) {
-      m.log_kbe[j][k] = std::log(m.kbe[j][k]);
       m.inv_bdc[j][k] = 1.0 / m.bdc[j][k];
+      const long double c = 1.0548L * std::pow((long double)m.kbe[j][k], -(long double)kOmegaSlow);
+      m.omega_hi[j][k] = (double)c;
+      m.omega_lo[j][k] = (double)(c - m.omega_hi[j][k]);
+      kbe_max = std::max(kbe_max, m.kbe[j][k]);
+    }
+  }
+  m.t_omega = (std::ldexp(1.0, kOmegaOctaves - 1) - 2) / kbe_max;
+  // of four s a step of 2^-40 apart the one whose s^2.1705 lies nearest to a double (Gal's accurate tables): its rounding
+  // then adds little to the error
+  for (int n = 0; n < kOmegaTable; ++n) {
+    const double mid = 1 + (2 * (n % 16) + 1) / 32.0;
+    double best = 1;
+    for (int q = 0; q < 4; ++q) {
+      const double s = std::ldexp(1 / mid * (1 + std::ldexp(q, -40)), 1 - n / 16);
+      const long double e = std::pow((long double)s, (long double)kOmegaPower);
+      const double err = std::fabs((double)(((double)e - e) / e));
+      if (err >= best) continue;
+      best = err;
+      m.omega_table[n][0] = s;
+      m.omega_table[n][1] = (double)e;
     }
   }
   m.has_transport = 1;
