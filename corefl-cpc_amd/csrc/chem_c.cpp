@@ -76,7 +76,7 @@ void chem_ensure_device(corefl_chem *c) {
                              std::to_string(c->mech.ns));
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   HIPCHK(hipMalloc(&c->mech_dev, sizeof(corefl::ChemMech)));
-  HIPCHK(hipMalloc(&c->counter, sizeof(int)));
+  HIPCHK(hipMalloc(&c->counter, 2 * sizeof(int)));
   HIPCHK(hipMalloc(&c->list_count, sizeof(int)));
   HIPCHK(hipMemcpy(c->mech_dev, &c->mech, sizeof(corefl::ChemMech), hipMemcpyHostToDevice));
   // the surrogate's projection tables, ready before any sub-step is captured into a graph

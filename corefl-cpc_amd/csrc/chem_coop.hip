@@ -446,7 +446,6 @@ __device__ __forceinline__ void row_attempt(const ChemMech &m, const MechLds &S,
   }
 }
 
-__global__ void k_zero_counter(int *p) { *p = 0; }
 
 __device__ __forceinline__ int work_count(const ChemBatch &b) { return b.list ? *b.n_list : b.n; }
 __device__ __forceinline__ int work_cell(const ChemBatch &b, int w) { return b.list ? b.list[w] : w; }
@@ -539,7 +538,6 @@ hipError_t launch_chem_coop(const ChemMech *mech_dev, int ns, const ChemBatch &b
   if (b.n == 0) return hipSuccess;
   if (threads != 64 && threads != 128 && threads != 256) return hipErrorInvalidValue;
   if (blocks < 1) return hipErrorInvalidValue;
-  k_zero_counter<<<1, 1, 0, s>>>(counter);
   k_chem_coop<9><<<blocks, threads, 0, s>>>(mech_dev, b, dt, rtol, atol, max_attempts, counter, resume ? 1 : 0);
   return hipGetLastError();
 }

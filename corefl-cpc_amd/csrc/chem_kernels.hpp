@@ -48,7 +48,7 @@ struct ChemLaunch {
 
 // e = sum_k Y_k h_k(T) - R T from T and rho Y (ConstVolumeReactor.cpp:60-68).
 hipError_t launch_chem_energy(const ChemMech *mech_dev, int ns, const ChemBatch &b, hipStream_t s);
-// One chemistry sub-step of length dt for every cell.  counter: device int used by the queue launches
+// One chemistry sub-step of length dt for every cell.  counter: two device ints used by the queue launches
 // (cleared by the launch itself).  Every mode gives the same result to rounding: mode 2 distributes the same
 // operations over lanes in the same order.
 hipError_t launch_chem_integrate(const ChemMech *mech_dev, int ns, const ChemBatch &b, double dt, double rtol,
@@ -57,7 +57,7 @@ hipError_t launch_chem_integrate(const ChemMech *mech_dev, int ns, const ChemBat
 hipError_t launch_chem_omega(const ChemMech *mech_dev, int ns, const ChemBatch &b, double *omega, hipStream_t s);
 hipError_t launch_chem_temperature(const ChemMech *mech_dev, int ns, const ChemBatch &b, hipStream_t s);
 // Cooperative integration (chem_coop.hip): work items of b (its list or all cells), fresh or resumed from the
-// hand-over state.
+// hand-over state.  counter: zero at the launch.
 hipError_t launch_chem_coop(const ChemMech *mech_dev, int ns, const ChemBatch &b, double dt, double rtol,
                             double atol, int max_attempts, int threads, int blocks, bool resume, int *counter,
                             hipStream_t s);

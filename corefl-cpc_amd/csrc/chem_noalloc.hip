@@ -19,7 +19,7 @@ constexpr long long kMaxCells = 1LL << 20;
 constexpr size_t kDoubles = sizeof(double) * (size_t)kMaxCells;
 constexpr size_t kInts = sizeof(int) * (size_t)kMaxCells;
 // Layout (byte offsets): h, tcur, elast (double per cell); steps, rejects, defer (int per cell); then the
-// work-queue counter and the hand-over count.  36 MiB + 256 B.
+// work-queue counters and the hand-over count.  36 MiB + 256 B.
 constexpr size_t kOffH = 0, kOffTcur = kDoubles, kOffElast = 2 * kDoubles, kOffSteps = 3 * kDoubles,
                  kOffRejects = kOffSteps + kInts, kOffDefer = kOffRejects + kInts, kOffCounter = kOffDefer + kInts,
                  kOffNDefer = kOffCounter + 128, kScratchBytes = kOffCounter + 256;
@@ -86,7 +86,7 @@ extern "C" int corefl_chem_integrate_noalloc(corefl_chem *c, long long n, const 
     b.n_defer = reinterpret_cast<int *>(base + kOffNDefer);
     int *counter = reinterpret_cast<int *>(base + kOffCounter);
     // every cell starts from the full sub-step (a zero carried step size), as after corefl_chem_set_cells;
-    // the launches clear the queue counter and the hand-over count themselves
+    // the launches clear the queue counters and the hand-over count themselves
     k_clear_doubles<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(b.h, (long)n);
     COREFL_HIPCHK(hipGetLastError());
     COREFL_HIPCHK(corefl::launch_chem_integrate(c->mech_dev, c->mech.ns, b, dt, rtol, atol, max_attempts, c->cfg,

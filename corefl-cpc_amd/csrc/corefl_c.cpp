@@ -441,13 +441,14 @@ struct corefl_ctx {
     }
   }
 
-  void enqueue_dt(hipStream_t s, int clip) {
+  // advance: the simulated time moves here, by the step that it yields
+  void enqueue_dt(hipStream_t s, int clip, int advance = 0) {
     for (auto &b : blocks) {
       if (ns && b.mix.mul) HIPCHK(corefl::launch_mix_transport(b.dev, b.mix, s));
       if (ns) HIPCHK(corefl::launch_mix_local_dt(b.dev, b.mix, scheme, parts + b.part_offset, s));
       else HIPCHK(corefl::launch_local_dt(b.dev, scheme, parts + b.part_offset, s));
     }
-    HIPCHK(corefl::launch_dt_reduce(parts, n_parts, dt_dev, time_dev, t_end, clip, s));
+    HIPCHK(corefl::launch_dt_reduce(parts, n_parts, dt_dev, time_dev, t_end, clip, advance, s));
   }
 
   // The viscous fluxes of every block (and their exchange for the collocated scheme) on the side stream, the
@@ -508,7 +509,7 @@ struct corefl_ctx {
       for (size_t q = 0; q < blocks.size(); ++q)
         HIPCHK(corefl::launch_sponge_mean(blocks[q].dev, 5 + ns, blocks[q].sponge_mean, sponge_iter,
                                           q + 1 == blocks.size(), s));
-    if (compute_dt) enqueue_dt(s, 1);
+    if (compute_dt) enqueue_dt(s, 1, 1);
     if (wu_method >= 0) {
       wu_step(s);
     } else {
@@ -516,7 +517,7 @@ struct corefl_ctx {
       for (int rk = 0; rk < 3; ++rk) stage(rk, s);
       if (strang) chem_substep(0.5, s);
     }
-    HIPCHK(corefl::launch_time_advance(time_dev, dt_dev, s));
+    if (!compute_dt) HIPCHK(corefl::launch_time_advance(time_dev, dt_dev, s));
     if (residual) {
       for (auto &b : blocks) HIPCHK(corefl::launch_residual_partial(b.dev, b.last, res_parts + 4 * b.res_offset, s));
       HIPCHK(corefl::launch_residual_finish(res_parts, n_res_parts, n_nodes_total, mon, s));

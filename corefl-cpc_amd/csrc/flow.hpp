@@ -101,11 +101,12 @@ hipError_t launch_update(const DevBlock &b, const Scheme &sc, int rk, const doub
 // Most planes one thread of the z-marching node kernels walks along k (fewer on small blocks).
 int march_planes();
 // CFL time step: per-workgroup partial minima into part[0 .. dt_partial_count(b)), then the global
-// minimum of n partials into dt_dev[0], clipped to t_end - time_dev[0] when clip != 0.
+// minimum of n partials into dt_dev[0], clipped to t_end - time_dev[0] when clip != 0; with advance != 0
+// time_dev[0] is moved by it in the same launch (4 us less than by launch_time_advance).
 int dt_partial_count(const DevBlock &b);
 hipError_t launch_local_dt(const DevBlock &b, const Scheme &sc, double *part, hipStream_t s);
-hipError_t launch_dt_reduce(const double *part, long n, double *dt_dev, const double *time_dev, double t_end,
-                            int clip, hipStream_t s);
+hipError_t launch_dt_reduce(const double *part, long n, double *dt_dev, double *time_dev, double t_end,
+                            int clip, int advance, hipStream_t s);
 hipError_t launch_time_advance(double *time_dev, const double *dt_dev, hipStream_t s);
 
 // Normal deviate of the inflow noise (host and device): a counter-based draw from (seed, application, node,

@@ -1175,8 +1175,8 @@ __global__ __launch_bounds__(256) void k_local_dt(DevBlock b, Scheme sc, double 
   }
 }
 
-__global__ __launch_bounds__(1024) void k_dt_reduce(const double *part, long n, double *dt, const double *time,
-                                                    double t_end, int clip) {
+__global__ __launch_bounds__(1024) void k_dt_reduce(const double *part, long n, double *dt, double *time,
+                                                    double t_end, int clip, int advance) {
   double m = 1e+6;
   for (long p = threadIdx.x; p < n; p += blockDim.x) m = fmin(m, part[p]);
   for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off, 64));
@@ -1189,6 +1189,7 @@ __global__ __launch_bounds__(1024) void k_dt_reduce(const double *part, long n, 
     for (int q = 1; q < (int)(blockDim.x / 64); ++q) r = fmin(r, wmin[q]);
     if (clip && time[0] + r > t_end) r = t_end - time[0];
     dt[0] = r;
+    if (advance) time[0] += r;
   }
 }
 
@@ -1429,9 +1430,9 @@ hipError_t launch_local_dt(const DevBlock &b, const Scheme &sc, double *part, hi
   return hipGetLastError();
 }
 
-hipError_t launch_dt_reduce(const double *part, long n, double *dt_dev, const double *time_dev, double t_end,
-                            int clip, hipStream_t s) {
-  k_dt_reduce<<<1, 1024, 0, s>>>(part, n, dt_dev, time_dev, t_end, clip);
+hipError_t launch_dt_reduce(const double *part, long n, double *dt_dev, double *time_dev, double t_end,
+                            int clip, int advance, hipStream_t s) {
+  k_dt_reduce<<<1, 1024, 0, s>>>(part, n, dt_dev, time_dev, t_end, clip, advance);
   return hipGetLastError();
 }
 
