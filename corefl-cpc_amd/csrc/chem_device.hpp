@@ -404,7 +404,9 @@ __device__ __forceinline__ OmegaNode omega_node(const ChemMech &m, double t, dou
 __device__ __forceinline__ double omega_d(const ChemMech &m, const OmegaNode &w, int a, int b) {
   const double kbe = m.kbe[a][b];
   const double x = __builtin_fma(w.t, kbe, kOmegaShift), xl = __builtin_fma(w.t, kbe, kOmegaShift - x);
-  const int n = (__double2hiint(x) >> 16) - 0x3FE0; // 0x3FE0: 1/2
+  // 0x3FE0: 1/2; the bound holds the index where a well depth of zero or less makes x negative or NaN (the pair's omega_hi
+  // or the series is NaN then, and so is the result)
+  const unsigned n = min((unsigned)(__double2hiint(x) >> 16) - 0x3FE0u, (unsigned)kOmegaTable - 1u);
   const double s = m.omega_table[n][0], e = m.omega_table[n][1];
   const double r = __builtin_fma(xl, s, __builtin_fma(x, s, -1.0));
   constexpr PowerSeries series(kOmegaPower);

@@ -4,8 +4,9 @@ import numpy as np
 import pytest
 
 import cases
+import chem_cases as CC
 import corefl
-from parity import make_mix_pair, rel_err
+from parity import make_mix_pair, make_solver, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +31,20 @@ def test_viscous_residual_over_temperatures(factor):
     assert np.max(err) < 1e-12
     dt = B.cfl_dt()
     assert abs(S.compute_dt() - dt) <= 1e-13 * dt
+
+
+@pytest.mark.parametrize("depth", ["0.000", "-97.53"])
+def test_well_depth_of_zero_or_less_gives_nan(depth, tmp_path):
+    """T* is infinite, negative or NaN: no place in the table, and not a number in the fluxes that use it."""
+    text = open(CC.TRAN_FILE).read()
+    line = next(l for l in text.split("\n") if l.startswith("N2 "))
+    path = tmp_path / "tran.dat"
+    path.write_text(text.replace(line, line.replace("97.530", depth)))
+    case = cases.reactive_box(N, recon=2, inviscid=4, temporal=3, reaction=0, visc=2)
+    assert CC.TRAN_FILE in case["setup"]
+    S = make_solver(dict(case, setup=case["setup"].replace(CC.TRAN_FILE, str(path))))
+    S.rhs()
+    S.sync()
+    dq = S.get(corefl.DQ).reshape(14, -1)
+    assert np.all(np.isfinite(dq[0]))
+    assert np.all(np.isnan(dq[4:]))
