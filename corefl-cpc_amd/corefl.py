@@ -25,7 +25,7 @@ SYMBOLS = (
     "corefl_chem_substep",
     "corefl_chem_create", "corefl_chem_create_mem", "corefl_chem_destroy", "corefl_chem_info", "corefl_chem_name",
     "corefl_chem_table", "corefl_chem_set_cells", "corefl_chem_set_cell_dt", "corefl_chem_get_cells", "corefl_chem_view_get",
-    "corefl_chem_source", "corefl_chem_integrate", "corefl_chem_set_launch", "corefl_chem_get_launch",
+    "corefl_chem_source", "corefl_chem_integrate", "corefl_chem_set_launch", "corefl_chem_get_launch", "corefl_chem_handed_over",
     "corefl_chem_autotune", "corefl_chem_synchronize", "corefl_chem_integrate_noalloc",
     "corefl_surrogate_n_params", "corefl_surrogate_create", "corefl_surrogate_destroy", "corefl_surrogate_set_params",
     "corefl_surrogate_get_params", "corefl_surrogate_set_scaling", "corefl_surrogate_set_transform",
@@ -130,6 +130,7 @@ def load_library(path=LIB_PATH):
     lib.corefl_chem_integrate.argtypes = [P, D, D, D, I, P]
     lib.corefl_chem_set_launch.argtypes = [P, I, I, I, I]
     lib.corefl_chem_get_launch.argtypes = [P, PI, PI, PI, PI]
+    lib.corefl_chem_handed_over.argtypes = [P, PI]
     lib.corefl_chem_autotune.argtypes = [P, D, D, D, I, I, ctypes.POINTER(D), I]
     lib.corefl_chem_synchronize.argtypes = [P]
     lib.corefl_chem_integrate_noalloc.argtypes = [P, LL, P, P, P, P, D, D, D, I, P]
@@ -447,7 +448,8 @@ class Chemistry:
 
     def set_launch(self, mode, threads=64, blocks=1024, budget=0):
         """mode 0: one thread per cell; 1: work queue; 2: cooperative (16 lanes per cell); 3: work queue for
-        at least `budget` attempts, then cooperative for the last cells.  A bool mode means 1 (True) or 0 (False)."""
+        at least `budget` attempts, then cooperative for the last cells.  All modes give the same bits.  A bool mode
+        means 1 (True) or 0 (False)."""
         _check(self._lib.corefl_chem_set_launch(self._ctx, int(mode), int(threads), int(blocks), int(budget)))
 
     def get_launch(self):
@@ -455,6 +457,12 @@ class Chemistry:
         _check(self._lib.corefl_chem_get_launch(self._ctx, ctypes.byref(q), ctypes.byref(t), ctypes.byref(b),
                                                 ctypes.byref(k)))
         return dict(queue=q.value, threads=t.value, blocks=b.value, budget=k.value)
+
+    def handed_over(self):
+        """Cells that the latest sub-step in mode 3 continued in the cooperative kernel."""
+        n = ctypes.c_int()
+        _check(self._lib.corefl_chem_handed_over(self._ctx, ctypes.byref(n)))
+        return n.value
 
     def autotune(self, dt, rtol=1e-6, atol=1e-8, max_attempts=100000, reps=1):
         """Time every candidate launch shape on the current batch; keeps the fastest.  Returns ms per

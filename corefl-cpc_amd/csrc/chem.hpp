@@ -53,6 +53,7 @@ struct ChemMech {
   // lanes take them (fall-off reactions last, so that a pass of 16 holds either kind), and the most species on a side
   ReacRecord rec[kMaxReac];
   int by_cost[kMaxReac], max_f, max_b;
+  int both_sides; // some reaction has a species on its left and on its right
   // fit ranges common to all species (common_range = 1), so that a wavefront whose temperatures lie on one side of the
   // middle reads one set of coefficients through scalar loads
   int common_range;

@@ -110,6 +110,7 @@ void chem_ensure_batch(corefl_chem *c, long long n) {
   HIPCHK(hipMalloc(&c->b.rejects, sizeof(int) * (size_t)n));
   HIPCHK(hipMalloc(&c->b.defer, sizeof(int) * (size_t)n));
   HIPCHK(hipMalloc(&c->b.n_defer, sizeof(int)));
+  HIPCHK(hipMemset(c->b.n_defer, 0, sizeof(int)));
   HIPCHK(hipMalloc(&c->b.tcur, d));
   HIPCHK(hipMalloc(&c->b.elast, d));
   HIPCHK(hipMalloc(&c->dtc, d));
@@ -356,6 +357,16 @@ int corefl_chem_get_launch(const corefl_chem *c, int *mode, int *threads, int *b
     if (threads) *threads = c->cfg.threads;
     if (blocks) *blocks = c->cfg.blocks;
     if (budget) *budget = c->cfg.budget;
+  });
+}
+
+int corefl_chem_handed_over(corefl_chem *c, int *n) {
+  return guarded([&] {
+    if (!c || !n) throw std::runtime_error("corefl_chem_handed_over: null argument");
+    *n = 0;
+    if (!c->b.n_defer) return;
+    HIPCHK(hipDeviceSynchronize());
+    HIPCHK(hipMemcpy(n, c->b.n_defer, sizeof(int), hipMemcpyDeviceToHost));
   });
 }
 

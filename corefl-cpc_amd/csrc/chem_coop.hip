@@ -19,8 +19,8 @@
 // An attempt of a wave takes 25 us alone on its SIMD and 37 us with a second one: the three sources 16, of which the
 // Jacobian 2.5, the factorisation 2, the solves 2.3, the temperatures 3.5.
 //
-// The operations are those of the one-lane attempt (chem_kernels.hip) in another order of summation: the two agree to
-// rounding.
+// The operations are those of the one-lane attempt (chem_kernels.hip), each sum in the same order, so that a cell gets the
+// same bits wherever it is integrated and whenever it is handed over.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -65,8 +65,8 @@ __device__ __forceinline__ void wave_sync() {
 
 constexpr int kPad = 16; // species index of an unused place on a reaction's side: concentration 1, g 0
 
-// The mechanism in LDS.  Species tables [field][species], reaction tables [field][place] and [place][species], places in
-// the order of ChemMech::by_cost.
+// The mechanism in LDS.  Species tables [field][species]; the tables of the rates [field][place], places in the order of
+// ChemMech::by_cost; the stoichiometry [reaction][species], since production is summed in the mechanism's order.
 struct MechLds {
   double lo[7][kMaxSpec], hi[7][kMaxSpec];
   double t_low[kMaxSpec], t_mid[kMaxSpec], t_high[kMaxSpec];
@@ -75,7 +75,7 @@ struct MechLds {
   double A[kMaxReac], b[kMaxReac], Ea[kMaxReac], A2[kMaxReac], b2[kMaxReac], Ea2[kMaxReac], troe[4][kMaxReac];
   double tb[kMaxSpec][kMaxReac];
   double dnu[kMaxReac][kMaxSpec], nf[kMaxReac][kMaxSpec], nb[kMaxReac][kMaxSpec];
-  int type[kMaxReac], rev[kMaxReac], iorder[kMaxReac];
+  int type[kMaxReac], rev[kMaxReac], iorder[kMaxReac], order[kMaxReac]; // order: the reaction of a place
   unsigned fsp[kMaxReac], bsp[kMaxReac];
   unsigned long long fnu[kMaxReac], bnu[kMaxReac];
 };
@@ -108,6 +108,7 @@ __device__ __forceinline__ void stage_mechanism(const ChemMech &m, MechLds &S) {
     S.Ea2[p] = q.Ea2;
 #pragma unroll
     for (int k = 0; k < 4; ++k) S.troe[k][p] = q.troe[k];
+    S.order[p] = r;
     S.type[p] = q.type;
     S.rev[p] = q.rev;
     S.iorder[p] = q.iorder;
@@ -120,11 +121,11 @@ __device__ __forceinline__ void stage_mechanism(const ChemMech &m, MechLds &S) {
     S.bnu[p] = q.bnu;
   }
   for (int q = threadIdx.x; q < m.nr * kMaxSpec; q += blockDim.x) {
-    const int p = q / kMaxSpec, n = q % kMaxSpec, r = m.by_cost[p];
-    S.dnu[p][n] = m.dnu[r][n];
-    S.nf[p][n] = m.nf[r][n];
-    S.nb[p][n] = m.nb[r][n];
-    S.tb[n][p] = m.tb[r][n];
+    const int p = q / kMaxSpec, n = q % kMaxSpec;
+    S.dnu[p][n] = m.dnu[p][n];
+    S.nf[p][n] = m.nf[p][n];
+    S.nb[p][n] = m.nb[p][n];
+    S.tb[n][p] = m.tb[m.by_cost[p]][n];
   }
 }
 
@@ -167,18 +168,26 @@ __device__ __forceinline__ double own_gibbs(const MechLds &S, int a, double t, d
 // enthalpy and heat capacity are those of its summed coefficients where all species share their fit range, else the sums
 // of the species' own.
 template<int NS>
-__device__ __forceinline__ double row_update_t(const ChemMech &m, const MechLds &S, int a, double t, double yk, double E) {
+__device__ __forceinline__ double row_update_t(const ChemMech &m, const MechLds &S, RowLds &X, int a, int gl, double t, double yk,
+                                               double E) {
   const double R = kRu * row_sum(yk * S.imw[a]), yr = yk * (kRu * S.imw[a]);
   double err = 1e+6, C[6];
   int side = -1;
+  X.c[gl] = yr; // free between two sources
+  wave_sync();
 #pragma unroll 1
   for (int it = 0; it < 100 && err > 1e-8; ++it) {
     double h, cp;
     if (m.common_range) {
       const int now = t < m.ct_mid ? 0 : 1;
       if (now != side) { // all lanes of a row alike
+        // lane q sums coefficient q over the species in their order, as the one-lane iteration does
+        const int q = gl < 6 ? gl : 5;
+        const double *c = now ? S.hi[q] : S.lo[q];
+        double d = 0;
 #pragma unroll
-        for (int q = 0; q < 6; ++q) C[q] = row_sum(yr * (now ? S.hi[q][a] : S.lo[q][a]));
+        for (int l = 0; l < NS; ++l) d = fma(X.c[l], c[l], d);
+        static_for<0, 6>([&](auto Q) { C[decltype(Q)::value] = row_bcast_c<decltype(Q)::value>(d); });
         side = now;
       }
       h_cp_fit(C, 1.0, t, fmin(fmax(t, m.ct_low), m.ct_high), h, cp);
@@ -192,10 +201,11 @@ __device__ __forceinline__ double row_update_t(const ChemMech &m, const MechLds 
       h = row_sum(h);
       cp = row_sum(cp);
     }
-    const double t1 = t - (h - R * t - E) / (cp - R);
+    const double t1 = t - (fma(-R, t, h) - E) / (cp - R);
     err = fabs(1 - t1 / t);
     t = t1;
   }
+  wave_sync();
   return t;
 }
 
@@ -213,49 +223,23 @@ __device__ __forceinline__ void reaction_rates(const ChemMech &m, const MechLds 
     for (int s = 0; s < most; ++s) {
       const int l = sp >> 8 * s & 255u, n = (short)(nu >> 16 * s & 65535u);
       const double x = X.c[l];
-      dg += X.g[l] * (sign * n);
+      dg = fma(X.g[l], sign * n, dg);
       if (n == 1) q *= x;
       else q *= int_pow(x, n);
     }
   };
   side(fsp, fnu, m.max_f, -1.0, q1);
   side(bsp, bnu, m.max_b, 1.0, q2);
-  double kf = arrhenius(lnT, iT, S.A[r], S.b[r], S.Ea[r]);
   double cc = 0;
   if (ty >= 4)
-    for (int l = 0; l < ns; ++l) cc += X.c[l] * S.tb[l][r];
-  if (ty == 3) {
-    kf += arrhenius(lnT, iT, A2, b2, Ea2);
-  } else if (ty == 4) {
-    kf *= cc;
-  } else if (ty > 4) {
-    const double klow = arrhenius(lnT, iT, A2, b2, Ea2), khigh = kf;
-    if (khigh < 1e-25 && klow < 1e-25) {
-      kf = 0;
-    } else {
-      const double pr = klow * cc / khigh;
-      double F = 1.0;
-      if (ty > 5) {
-        double fc = (1 - S.troe[0][r]) * exp(-t / S.troe[1][r]) + S.troe[0][r] * exp(-t / S.troe[2][r]);
-        if (ty == 7) fc += exp(-S.troe[3][r] * iT);
-        const double lfc = log10(fc);
-        const double cq = -0.4 - 0.67 * lfc, nq = 0.75 - 1.27 * lfc;
-        const double lpr = log10(pr);
-        const double tmp = (lpr + cq) / (nq - 0.14 * (lpr + cq));
-        F = exp(2.302585092994046 * lfc / (1.0 + tmp * tmp)); // 10^x
-      }
-      kf = khigh * pr / (1.0 + pr) * F;
-    }
-  }
+    for (int l = 0; l < ns; ++l) cc = fma(X.c[l], S.tb[l][r], cc);
+  const double kf = forward_rate(ty, S.A[r], S.b[r], S.Ea[r], A2, b2, Ea2, t, lnT, iT, cc, [&](int k) { return S.troe[k][r]; });
   double kb = 0;
   if (ty != 0 && rev == 1) {
     kb = arrhenius(lnT, iT, A2, b2, Ea2);
     if (ty == 4) kb *= cc;
   }
-  if (m.need_gibbs && ty != 0 && ty != 2) {
-    const double tp = kPatm / kRu * 1e-3 * iT, itp = kRu / kPatm * 1e+3 * t;
-    kb = kf * exp(dg) * int_pow(order < 0 ? tp : itp, order < 0 ? -order : order);
-  }
+  if (m.need_gibbs && ty != 0 && ty != 2) kb = gibbs_reverse(kf, dg, order, kPatm / kRu * 1e-3 * iT, kRu / kPatm * 1e+3 * t);
   q1o = q1 * kf;
   q2o = q2 * kb;
 }
@@ -276,14 +260,17 @@ __device__ __forceinline__ double row_source(const ChemMech &m, const MechLds &S
     if (r < nr) {
       double q1, q2;
       reaction_rates(m, S, X, r, NS, t, lnT, iT, q1, q2);
-      X.q1[r] = jac ? q1 : q1 - q2;
-      X.q2[r] = q2;
+      const int o = S.order[r];
+      X.q1[o] = jac ? q1 : q1 - q2;
+      X.q2[o] = q2;
     }
   }
   wave_sync();
   const double scale = 1e+3 * S.mw[a];
   double w = 0;
-  if (!jac) {
+  if (!jac && m.both_sides) { // a species' two coefficients one after the other, as the one-lane source adds them
+    for (int r = 0; r < nr; ++r) w = fma(S.nb[r][a], X.q1[r], fma(-S.nf[r][a], X.q1[r], w));
+  } else if (!jac) {
 #pragma unroll 8
     for (int r = 0; r < nr; ++r) w = fma(S.dnu[r][a], X.q1[r], w);
   } else {
@@ -293,9 +280,12 @@ __device__ __forceinline__ double row_source(const ChemMech &m, const MechLds &S
 #pragma unroll 2
     for (int r = 0; r < nr; ++r) {
       const double q1 = X.q1[r], q2 = X.q2[r], dn = S.dnu[r][a];
-      const double v = S.nf[r][a] * q1 - S.nb[r][a] * q2;
-      w = fma(dn, q1 - q2, w);
-      static_for<0, NS>([&](auto N) { Jrow[decltype(N)::value] += dn * row_bcast_c<decltype(N)::value>(v); });
+      const double nf = S.nf[r][a], nb = S.nb[r][a], qn = q1 - q2, v = fma(nf, q1, -(nb * q2));
+      w = fma(nb, qn, fma(-nf, qn, w));
+      static_for<0, NS>([&](auto N) {
+        constexpr int n = decltype(N)::value;
+        Jrow[n] = fma(dn, row_bcast_c<n>(v), Jrow[n]);
+      });
     }
     const double inv = ya > 1e-30 ? 1.0 / ya : 0.0;
     static_for<0, NS>([&](auto N) {
@@ -346,7 +336,7 @@ template<int NS> __device__ __forceinline__ int row_lu(double *row, int a) {
       const double l = row[k] * inv;
       row[k] = l;
 #pragma unroll
-      for (int t = k + 1; t < NS; ++t) row[t] -= l * prow[t];
+      for (int t = k + 1; t < NS; ++t) row[t] = fma(-l, prow[t], row[t]);
     } else if (a == k) {
       row[k] = inv;
     }
@@ -367,7 +357,7 @@ template<int NS> __device__ __forceinline__ double row_solve(const double *row, 
   static_for<0, NS - 1>([&](auto T) {
     constexpr int t = decltype(T)::value;
     const double bt = row_bcast_c<t>(b);
-    const double nb = b - row[t] * bt;
+    const double nb = fma(-row[t], bt, b);
     b = a > t ? nb : b;
   });
   if (a == NS - 1) b *= row[NS - 1];
@@ -377,7 +367,7 @@ template<int NS> __device__ __forceinline__ double row_solve(const double *row, 
     constexpr int r = NS - 2 - decltype(I)::value;
     double v = b;
 #pragma unroll
-    for (int t = r + 1; t < NS; ++t) v -= row[t] * fin[t];
+    for (int t = r + 1; t < NS; ++t) v = fma(-row[t], fin[t], v);
     v *= row[r];
     b = a == r ? v : b;
     fin[r] = row_bcast_c<r>(b);
@@ -407,25 +397,28 @@ __device__ __forceinline__ void row_attempt(const ChemMech &m, const MechLds &S,
 #pragma unroll 1
   for (int st = 0; st < 5; ++st) {
     if (st != 3) { // the fourth stage takes the third's source
-      if (st < 4) ys = s.y + hs * (kStageA[st][0] * k1 + kStageA[st][1] * k2);
+      if (st < 4) ys = stage_state(st, s.y, hs, k1, k2);
       // st 4: ys is the new state, and an accepted step gets its temperature from the old one
-      if (st > 0 && (st < 4 || err <= 1)) Ts = row_update_t<NS>(m, S, a, st == 4 ? s.T : Ts, own ? ys * irho : 0.0, s.E);
+      if (st > 0 && (st < 4 || err <= 1)) Ts = row_update_t<NS>(m, S, X, a, gl, st == 4 ? s.T : Ts, own ? ys * irho : 0.0, s.E);
       if (st == 4) break;
       w = row_source<NS>(m, S, X, a, gl, Ts, ys, st == 0, Jrow);
       if (st == 0) {
 #pragma unroll
-        for (int n = 0; n < NS; ++n) Jrow[n] = -hs * G * Jrow[n] + (n == a ? 1.0 : 0.0);
+        for (int n = 0; n < NS; ++n) {
+          const double j = -hs * G * Jrow[n];
+          Jrow[n] = n == a ? j + 1.0 : j;
+        }
         src = row_lu<NS>(Jrow, a);
       }
     }
-    const double c = kStageG[st][0] * k1 + kStageG[st][1] * k2 + kStageG[st][2] * k3;
+    const double c = stage_sum(st, k1, k2, k3);
     const double k = row_solve<NS>(Jrow, a, src, w + c) - c;
     if (st == 0) k1 = k;
     else if (st == 1) k2 = k;
     else if (st == 2) k3 = k;
     else {
-      ys = s.y + hs * (B1 * k1 + B2 * k2 + B4 * k);
-      const double dy = hs * (E1 * k1 + E2 * k2 + E3 * k3 + E4 * k) / (rtol * ys + atol);
+      ys = new_state(s.y, hs, k1, k2, k);
+      const double dy = error_term(ys, hs, k1, k2, k3, k, rtol, atol);
       err = sqrt(row_sum(own ? dy * dy : 0.0) / NS);
     }
   }

@@ -12,6 +12,11 @@
 namespace corefl {
 namespace chemdev {
 
+// The one-lane and the cooperative integrator hand cells to one another at moments that scheduling sets, so both have to
+// give a cell the same bits: what they share is written once, here and in rok4e.hpp, with every fused multiply-add spelled
+// out and every sum in one order, and the files of both are compiled without contraction (but for the differences
+// x -= a b marked so, where a negation written out would be an instruction of its own).
+
 constexpr double kRu = 8314.462618, kPatm = 101325.0;
 // constant divisions of the polynomial fits as products (a few ulp from the divided form)
 constexpr double kThird = 1.0 / 3.0, kSixth = 1.0 / 6.0, kTwelfth = 1.0 / 12.0;
@@ -69,7 +74,7 @@ template<int NS> __device__ __forceinline__ void h_cp(const ChemMech &m, double 
 // species whose fit range holds t; the logarithms of the range ends are tabulated.
 __device__ __forceinline__ double gibbs_fit(const double *c, double tt, double lt, double itt) {
   const double p = fma(tt, fma(tt, fma(tt, c[4] * 0.05, c[3] * kTwelfth), c[2] * kSixth), 0.5 * c[1]);
-  return fma(c[0], 1.0 - lt, fma(c[5], itt, -c[6])) - tt * p;
+  return fma(-tt, p, fma(c[0], 1.0 - lt, fma(c[5], itt, -c[6])));
 }
 
 template<int NS>
@@ -99,7 +104,7 @@ __device__ __forceinline__ void gibbs(const ChemMech &m, double t, double lnT, d
 // A T^b exp(-Ea/T) as A exp(b ln T - Ea/T): one exponential per rate instead of a power and an exponential
 // (the same value up to rounding).
 __device__ __forceinline__ double arrhenius(double lnT, double iT, double A, double b, double Ea) {
-  return A * exp(b * lnT - Ea * iT);
+  return A * exp(fma(b, lnT, -(Ea * iT)));
 }
 
 // x^k for an integer k (reaction orders and stoichiometric coefficients are integers: the parser rejects
@@ -109,6 +114,87 @@ __device__ __forceinline__ double int_pow(double x, int k) {
   double r = 1.0;
   for (int q = 0; q < n; ++q) r *= x;
   return k < 0 ? 1.0 / r : r;
+}
+
+// N sums over the species as the cooperative kernel's 16 lanes form them: the two halves, then quarters, pairs and
+// neighbours (the places beyond NS hold zeros there).  term(l, v) gives species l's terms; they are taken as they are
+// added, so that few are alive at a time.
+template<int NS, int N, class F> __device__ __forceinline__ void species_sums(F &&term, double (&sum)[N]) {
+  static_assert(NS <= 16);
+  auto eighth = [&](int i, double (&v)[N]) { // places i and i + 8
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = 0.0;
+    if (i < NS) term(i, v);
+    if (i + 8 < NS) {
+      double x[N];
+      term(i + 8, x);
+#pragma unroll
+      for (int q = 0; q < N; ++q) v[q] += x[q];
+    }
+  };
+  auto quarter = [&](int i, double (&v)[N]) {
+    double x[N];
+    eighth(i, v);
+    eighth(i + 4, x);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] += x[q];
+  };
+  auto half = [&](int i, double (&v)[N]) {
+    double x[N];
+    quarter(i, v);
+    quarter(i + 2, x);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] += x[q];
+  };
+  double x[N];
+  half(0, sum);
+  half(1, x);
+#pragma unroll
+  for (int q = 0; q < N; ++q) sum[q] += x[q];
+}
+template<int NS> __device__ __forceinline__ double species_sum(const double *x) {
+  double sum[1];
+  species_sums<NS>([&](int l, double (&v)[1]) { v[0] = x[l]; }, sum);
+  return sum[0];
+}
+
+// Forward rate constant of a reaction of type ty: cc its third-body concentration (types 4 and up), troe(k) its fall-off
+// parameters.
+template<class Troe>
+__device__ __forceinline__ double forward_rate(int ty, double A, double b, double Ea, double A2, double b2, double Ea2, double t,
+                                               double lnT, double iT, double cc, Troe &&troe) {
+  double kf = arrhenius(lnT, iT, A, b, Ea);
+  if (ty == 3) {
+    kf += arrhenius(lnT, iT, A2, b2, Ea2);
+  } else if (ty == 4) {
+    kf *= cc;
+  } else if (ty > 4) {
+    const double klow = arrhenius(lnT, iT, A2, b2, Ea2), khigh = kf;
+    if (khigh < 1e-25 && klow < 1e-25) {
+      kf = 0;
+    } else {
+      const double pr = klow * cc / khigh;
+      double F = 1.0;
+      if (ty > 5) {
+        const double a = troe(0);
+        double fc = fma(1 - a, exp(-t / troe(1)), a * exp(-t / troe(2)));
+        if (ty == 7) fc += exp(-troe(3) * iT);
+        const double lfc = log10(fc);
+        const double cq = fma(-0.67, lfc, -0.4), nq = fma(-1.27, lfc, 0.75);
+        const double lpr = log10(pr);
+        const double tmp = (lpr + cq) / fma(-0.14, lpr + cq, nq);
+        F = exp(2.302585092994046 * lfc / fma(tmp, tmp, 1.0)); // 10^x
+      }
+      kf = khigh * pr / (1.0 + pr) * F;
+    }
+  }
+  return kf;
+}
+
+// Reverse rate constant from the forward one: dg the sum of nu g / (R T) over the products less that over the reactants,
+// tp and itp p_atm / (R T) in kmol/m^3 and its reciprocal; kf / (tp^order exp(-dg)), without dividing.
+__device__ __forceinline__ double gibbs_reverse(double kf, double dg, int order, double tp, double itp) {
+  return kf * exp(dg) * int_pow(order < 0 ? tp : itp, order < 0 ? -order : order);
 }
 
 // Chemical source omega [kg/(m^3 s)] of one cell (FiniteRateChem.cu:1466-1605).  With JAC, also the
@@ -133,11 +219,10 @@ __device__ __forceinline__ void source(const ChemMech &m, double t, const double
 #pragma unroll
       for (int q = 0; q < NS * NS; ++q) J[q] = 0;
   }
+  const double lnT = log(t), iT = 1.0 / t;
   // Equilibrium constants are needed unless every reversible reaction carries explicit REV parameters
   // (FiniteRateChem.cu:1519-1557); then they are applied to every reaction of type other than 0 and 2.
-  const double lnT = log(t), iT = 1.0 / t;
   if (m.need_gibbs) gibbs<NS>(m, t, lnT, iT, g);
-  // p_atm / (R T) in kmol/m^3 and its reciprocal
   const double tp = kPatm / kRu * 1e-3 * iT, itp = kRu / kPatm * 1e+3 * t;
   for (int r = 0; r < m.nr; ++r) {
     const ReacRecord q = m.rec[r];
@@ -145,38 +230,15 @@ __device__ __forceinline__ void source(const ChemMech &m, double t, const double
     const int nfs = q.n_sides & 255, nbs = q.n_sides >> 8;
     auto sp = [](unsigned s, int k) { return (int)(s >> 8 * k & 255u); };
     auto nu = [](unsigned long long s, int k) { return (int)(short)(s >> 16 * k & 65535u); };
-    double kf = arrhenius(lnT, iT, q.A, q.b, q.Ea);
     double cc = 0;
     if (ty >= 4) {
       double tb[NS];
 #pragma unroll
       for (int l = 0; l < NS; ++l) tb[l] = m.tb[r][l];
 #pragma unroll
-      for (int l = 0; l < NS; ++l) cc += c[l] * tb[l];
+      for (int l = 0; l < NS; ++l) cc = fma(c[l], tb[l], cc);
     }
-    if (ty == 3) {
-      kf += arrhenius(lnT, iT, q.A2, q.b2, q.Ea2);
-    } else if (ty == 4) {
-      kf *= cc;
-    } else if (ty > 4) {
-      const double klow = arrhenius(lnT, iT, q.A2, q.b2, q.Ea2), khigh = kf;
-      if (khigh < 1e-25 && klow < 1e-25) {
-        kf = 0;
-      } else {
-        const double pr = klow * cc / khigh;
-        double F = 1.0;
-        if (ty > 5) {
-          double fc = (1 - q.troe[0]) * exp(-t / q.troe[1]) + q.troe[0] * exp(-t / q.troe[2]);
-          if (ty == 7) fc += exp(-q.troe[3] * iT);
-          const double lfc = log10(fc);
-          const double cq = -0.4 - 0.67 * lfc, nq = 0.75 - 1.27 * lfc;
-          const double lpr = log10(pr);
-          const double tmp = (lpr + cq) / (nq - 0.14 * (lpr + cq));
-          F = exp(2.302585092994046 * lfc / (1.0 + tmp * tmp)); // 10^x
-        }
-        kf = khigh * pr / (1.0 + pr) * F;
-      }
-    }
+    const double kf = forward_rate(ty, q.A, q.b, q.Ea, q.A2, q.b2, q.Ea2, t, lnT, iT, cc, [&](int k) { return q.troe[k]; });
     double kb = 0;
     if (ty != 0 && q.rev == 1) {
       kb = arrhenius(lnT, iT, q.A2, q.b2, q.Ea2);
@@ -184,10 +246,9 @@ __device__ __forceinline__ void source(const ChemMech &m, double t, const double
     }
     if (m.need_gibbs && ty != 0 && ty != 2) {
       double dg = 0;
-      for (int s = 0; s < nbs; ++s) dg += g[sp(q.bsp, s)] * nu(q.bnu, s);
-      for (int s = 0; s < nfs; ++s) dg -= g[sp(q.fsp, s)] * nu(q.fnu, s);
-      // kf / ((p_atm / R T)^order exp(-dg)), without dividing
-      kb = kf * exp(dg) * int_pow(q.iorder < 0 ? tp : itp, q.iorder < 0 ? -q.iorder : q.iorder);
+      for (int s = 0; s < nfs; ++s) dg = fma(g[sp(q.fsp, s)], -(double)nu(q.fnu, s), dg);
+      for (int s = 0; s < nbs; ++s) dg = fma(g[sp(q.bsp, s)], (double)nu(q.bnu, s), dg);
+      kb = gibbs_reverse(kf, dg, q.iorder, tp, itp);
     }
     double q1 = 1.0, q2 = ty != 0 ? 1.0 : 0.0;
     for (int s = 0; s < nfs; ++s) q1 *= int_pow(c[sp(q.fsp, s)], nu(q.fnu, s));
@@ -199,13 +260,13 @@ __device__ __forceinline__ void source(const ChemMech &m, double t, const double
     for (int s = 0; s < nfs; ++s) {
       const int l = sp(q.fsp, s);
       const double n = nu(q.fnu, s);
-      net[l] -= qn * n;
+      net[l] = fma(-n, qn, net[l]);
       if constexpr (WD) de[l] += q1 * n;
     }
     for (int s = 0; s < nbs; ++s) {
       const int l = sp(q.bsp, s);
       const double n = nu(q.bnu, s);
-      net[l] += qn * n;
+      net[l] = fma(n, qn, net[l]);
       if constexpr (WD) de[l] += q2 * n;
     }
     if constexpr (JAC) {
@@ -215,7 +276,7 @@ __device__ __forceinline__ void source(const ChemMech &m, double t, const double
       double v[NS], dn[NS];
 #pragma unroll
       for (int n = 0; n < NS; ++n) {
-        v[n] = m.nf[r][n] * q1 - m.nb[r][n] * q2;
+        v[n] = fma(m.nf[r][n], q1, -(m.nb[r][n] * q2));
         dn[n] = m.dnu[r][n];
       }
 #pragma unroll
@@ -223,7 +284,7 @@ __device__ __forceinline__ void source(const ChemMech &m, double t, const double
         if (!(am >> a & 1u)) continue;
 #pragma unroll
         for (int n = 0; n < NS; ++n)
-          if (um >> n & 1u) J[a * NS + n] += dn[a] * v[n];
+          if (um >> n & 1u) J[a * NS + n] = fma(dn[a], v[n], J[a * NS + n]);
       }
     }
   }
@@ -245,6 +306,7 @@ __device__ __forceinline__ void source(const ChemMech &m, double t, const double
 
 // Doolittle LU with partial pivoting, row-major (ConstVolumeReactor.cpp:1231-1262), and its solve.
 template<int NS> __device__ __forceinline__ void lu(double *a, int *piv) {
+#pragma clang fp contract(fast)
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
     // first row of largest |a[r][k]|; the running maximum keeps every array index static, so the matrix
@@ -290,6 +352,7 @@ template<int NS> __device__ __forceinline__ void lu(double *a, int *piv) {
 }
 
 template<int NS> __device__ __forceinline__ void lu_solve(const double *a, const int *piv, double *b) {
+#pragma clang fp contract(fast)
 #pragma unroll
   for (int r = 0; r < NS; ++r) {
     if (__any(piv[r] != r))
@@ -347,7 +410,7 @@ __device__ __forceinline__ double newton_t(const ChemMech &m, double t, const do
       }
       double h, cp;
       h_cp_fit(C, 1.0, t, fmin(fmax(t, m.ct_low), m.ct_high), h, cp);
-      const double t1 = t - (h - R * t - E) / (cp - R);
+      const double t1 = t - (fma(-R, t, h) - E) / (cp - R);
       err = fabs(1 - t1 / t);
       t = t1;
     }
@@ -355,14 +418,13 @@ __device__ __forceinline__ double newton_t(const ChemMech &m, double t, const do
   }
 #pragma unroll 1
   for (; it < most && err > tol; ++it) {
-    double h[NS], cp[NS], cpt = 0, hh = 0;
-    h_cp<NS>(m, t, h, cp);
-#pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      cpt += cp[l] * yk[l];
-      hh += h[l] * yk[l];
-    }
-    const double t1 = t - (hh - R * t - E) / (cpt - R);
+    double hc[2];
+    species_sums<NS>([&](int l, double (&v)[2]) {
+      const double lo = m.t_low[l], hi = m.t_high[l], tt = t < lo ? lo : (t > hi ? hi : t);
+      const bool low = t < lo || (!(t > hi) && t < m.t_mid[l]);
+      h_cp_fit(low ? m.lo[l] : m.hi[l], yk[l] * (kRu * m.imw[l]), t, tt, v[0], v[1]);
+    }, hc);
+    const double t1 = t - (fma(-R, t, hc[0]) - E) / (hc[1] - R);
     err = fabs(1 - t1 / t);
     t = t1;
   }
@@ -371,10 +433,10 @@ __device__ __forceinline__ double newton_t(const ChemMech &m, double t, const do
 
 // T at fixed specific internal energy E (ConstVolumeReactor.cpp:970-995).
 template<int NS> __device__ __forceinline__ double update_t(const ChemMech &m, double t, const double *yk, double E) {
-  double imw = 0;
+  double x[NS];
 #pragma unroll
-  for (int l = 0; l < NS; ++l) imw += yk[l] * m.imw[l];
-  return newton_t<NS>(m, t, yk, kRu * imw, E, 1e-8, 100);
+  for (int l = 0; l < NS; ++l) x[l] = yk[l] * m.imw[l];
+  return newton_t<NS>(m, t, yk, kRu * species_sum<NS>(x), E, 1e-8, 100);
 }
 
 // The coefficients of (1 + r)^-power.

@@ -55,11 +55,9 @@ __device__ __forceinline__ void rok4e_attempt(const ChemMech *mp, Cell<NS> &s, d
   for (int st = 0; st < 5; ++st) {
     const ChemMech &m = opaque(mp);
     if (st != 3) { // the fourth stage takes the third's source
-      if (st < 4) {
-        const double a1 = hs * kStageA[st][0], a2 = hs * kStageA[st][1];
+      if (st < 4)
 #pragma unroll
-        for (int l = 0; l < NS; ++l) ys[l] = s.y[l] + (a1 * k1[l] + a2 * k2[l]);
-      }
+        for (int l = 0; l < NS; ++l) ys[l] = stage_state(st, s.y[l], hs, k1[l], k2[l]);
       // st 4: ys is the new state, and an accepted step gets its temperature from the old one
       if (st > 0 && (st < 4 || err <= 1)) {
         double yk[NS];
@@ -77,13 +75,12 @@ __device__ __forceinline__ void rok4e_attempt(const ChemMech *mp, Cell<NS> &s, d
         lu<NS>(J, piv);
       }
     }
-    const double g1 = kStageG[st][0], g2 = kStageG[st][1], g3 = kStageG[st][2];
     double k[NS];
 #pragma unroll
-    for (int l = 0; l < NS; ++l) k[l] = w[l] + (g1 * k1[l] + g2 * k2[l] + g3 * k3[l]);
+    for (int l = 0; l < NS; ++l) k[l] = w[l] + stage_sum(st, k1[l], k2[l], k3[l]);
     lu_solve<NS>(J, piv, k);
 #pragma unroll
-    for (int l = 0; l < NS; ++l) k[l] -= g1 * k1[l] + g2 * k2[l] + g3 * k3[l];
+    for (int l = 0; l < NS; ++l) k[l] -= stage_sum(st, k1[l], k2[l], k3[l]);
     if (st == 0) {
 #pragma unroll
       for (int l = 0; l < NS; ++l) k1[l] = k[l];
@@ -94,13 +91,14 @@ __device__ __forceinline__ void rok4e_attempt(const ChemMech *mp, Cell<NS> &s, d
 #pragma unroll
       for (int l = 0; l < NS; ++l) k3[l] = k[l];
     } else {
+      double d2[NS];
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        ys[l] = s.y[l] + hs * (B1 * k1[l] + B2 * k2[l] + B4 * k[l]);
-        const double dy = hs * (E1 * k1[l] + E2 * k2[l] + E3 * k3[l] + E4 * k[l]) / (rtol * ys[l] + atol);
-        err += dy * dy;
+        ys[l] = new_state(s.y[l], hs, k1[l], k2[l], k[l]);
+        const double dy = error_term(ys[l], hs, k1[l], k2[l], k3[l], k[l], rtol, atol);
+        d2[l] = dy * dy;
       }
-      err = sqrt(err / NS);
+      err = sqrt(species_sum<NS>(d2) / NS);
     }
   }
   double hstar = hs;
@@ -176,7 +174,8 @@ template<int NS> __device__ __forceinline__ void store_partial(const ChemBatch &
 // budget > 0: a cell still unfinished after `budget` attempts is handed over (appended to b.defer) once fewer than 3/16
 // of the launch's lanes hold a cell.  An attempt of every cell takes 100 us here whatever their number up to one per
 // lane (65536 lanes), and in the cooperative kernel 60 us for every 8192 cells, so the lines cross near 13000 cells;
-// below, its shorter attempt counts.  (200003 igniting cells, 5.6 attempts on average and 123 at most: 5.8 ms, 6.7 with
+// below, its shorter attempt counts.  When that is reached depends on how waves are scheduled; a cell's bits do not, since
+// both kernels round alike.  (200003 igniting cells, 5.6 attempts on average and 123 at most: 5.8 ms, 6.7 with
 // every cell handed over after its fourth attempt.)
 template<int NS>
 __global__ __launch_bounds__(256) void k_chem_queue(const ChemMech *__restrict__ mp, ChemBatch b, double dt,
@@ -273,10 +272,10 @@ template<int NS> __global__ __launch_bounds__(256) void k_chem_energy(const Chem
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
     const double y = b.rhoY[(long)l * b.n + c] * irho;
-    e += h[l] * y;
-    imw += y * m.imw[l];
+    e = fma(h[l], y, e);
+    imw = fma(y, m.imw[l], imw);
   }
-  b.e[c] = e - kRu * imw * t;
+  b.e[c] = fma(-kRu * imw, t, e);
 }
 
 // One launch for all counters of a sub-step (they were three, of 4.9 us each).

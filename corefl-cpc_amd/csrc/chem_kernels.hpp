@@ -49,8 +49,8 @@ struct ChemLaunch {
 // e = sum_k Y_k h_k(T) - R T from T and rho Y (ConstVolumeReactor.cpp:60-68).
 hipError_t launch_chem_energy(const ChemMech *mech_dev, int ns, const ChemBatch &b, hipStream_t s);
 // One chemistry sub-step of length dt for every cell.  counter: two device ints used by the queue launches
-// (cleared by the launch itself).  Every mode gives the same result to rounding: mode 2 distributes the same
-// operations over lanes in the same order.
+// (cleared by the launch itself).  Every mode gives the same bits: mode 2 distributes the same operations over lanes,
+// each sum in the same order, so that it does not matter when mode 3 hands a cell over.
 hipError_t launch_chem_integrate(const ChemMech *mech_dev, int ns, const ChemBatch &b, double dt, double rtol,
                                  double atol, int max_attempts, const ChemLaunch &cfg, int *counter,
                                  hipStream_t s);

@@ -345,7 +345,7 @@ ChemMech parse_mechanism(const std::string &mech_text, const std::string &therm_
     pack(m.nfs[r], m.fsp[r], m.fnu[r], q.fsp, q.fnu);
     pack(m.nbs[r], m.bsp[r], m.bnu[r], q.bsp, q.bnu);
   }
-  m.max_f = m.max_b = 0;
+  m.max_f = m.max_b = m.both_sides = 0;
   int at = 0;
   for (int falloff = 0; falloff < 2; ++falloff)
     for (int r = 0; r < nr; ++r)
@@ -353,6 +353,8 @@ ChemMech parse_mechanism(const std::string &mech_text, const std::string &therm_
   for (int r = 0; r < nr; ++r) {
     m.max_f = std::max(m.max_f, m.nfs[r]);
     m.max_b = std::max(m.max_b, m.nbs[r]);
+    for (int k = 0; k < m.ns; ++k)
+      if (m.nf[r][k] != 0 && m.nb[r][k] != 0) m.both_sides = 1;
   }
   m.common_range = 1;
   for (int k = 1; k < m.ns; ++k)

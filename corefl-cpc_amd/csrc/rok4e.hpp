@@ -20,10 +20,25 @@ __constant__ const double kStageG[4][3] = {{0, 0, 0}, {G21, 0, 0}, {G31, G32, 0}
 // A step whose size h satisfies kStretch h >= (time left in the interval) is taken to the interval's end.
 constexpr double kStretch = 1.05;
 
+// A stage's state, the sum of earlier stages in its right-hand side, the new state and one species' term of the error
+// estimate, one rounding for both integrators.
+__device__ __forceinline__ double stage_state(int st, double y, double hs, double k1, double k2) {
+  return fma(hs, fma(kStageA[st][0], k1, kStageA[st][1] * k2), y);
+}
+__device__ __forceinline__ double stage_sum(int st, double k1, double k2, double k3) {
+  return fma(kStageG[st][0], k1, fma(kStageG[st][1], k2, kStageG[st][2] * k3));
+}
+__device__ __forceinline__ double new_state(double y, double hs, double k1, double k2, double k4) {
+  return fma(hs, fma(B1, k1, fma(B2, k2, B4 * k4)), y);
+}
+__device__ __forceinline__ double error_term(double y, double hs, double k1, double k2, double k3, double k4, double rtol, double atol) {
+  return hs * fma(E1, k1, fma(E2, k2, fma(E3, k3, E4 * k4))) / fma(rtol, y, atol);
+}
+
 // The PI controller's step factor after the first step, 0.8 err_last^0.1 (err + 1e-20)^-0.175 in [0.2, 5], its two powers
 // as one exponential of logarithms.
 __device__ __forceinline__ double step_factor(double err_last, double err) {
-  return fmin(5.0, fmax(0.2, 0.8 * exp(0.1 * log(err_last) - 0.175 * log(err + 1e-20))));
+  return fmin(5.0, fmax(0.2, 0.8 * exp(fma(0.1, log(err_last), -0.175 * log(err + 1e-20)))));
 }
 
 } // namespace rok4e

@@ -244,10 +244,14 @@ int corefl_chem_integrate(corefl_chem *chem, double dt, double rtol, double atol
  * thread, src/FiniteRateChem.cu:1388).  mode 0: one thread per cell; 1: persistent waves fetching cells
  * from a device counter, `blocks` workgroups; 2: persistent waves integrating four cells at a time, 16 lanes
  * per cell (lower latency per step attempt, for stiff cells); 3: mode 1 for at least `budget` attempts per
- * cell, the cells unfinished when few are left then continued by mode 2.  All modes give the same result to rounding.
+ * cell, the cells unfinished when few are left then continued by mode 2.  All modes give the same bits, so it does not
+ * matter that the moment of a hand-over depends on how waves are scheduled.
  * threads is 64, 128 or 256; budget is used by mode 3 only. */
 int corefl_chem_set_launch(corefl_chem *chem, int mode, int threads, int blocks, int budget);
 int corefl_chem_get_launch(const corefl_chem *chem, int *mode, int *threads, int *blocks, int *budget);
+/* Cells that the context's latest sub-step in mode 3 continued by mode 2 (0 before the first).  Waits for the device.
+ * No reference counterpart. */
+int corefl_chem_handed_over(corefl_chem *chem, int *n);
 /* Times corefl_chem_integrate(dt, rtol, atol, max_attempts) on the current batch for each candidate launch
  * shape (mode 0 with 64/128/256 threads; mode 1 with 64/128/256 threads x 4/8/16 waves per CU; mode 2 at
  * 4 and 8 waves per CU; mode 3 with budgets 4 and 16), `reps` runs each from the same saved state, keeps the

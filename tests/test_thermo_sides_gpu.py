@@ -9,13 +9,18 @@ import corefl
 pytestmark = pytest.mark.gpu
 
 
-def mechanism(common):
-    """The H2/air mechanism; common False: one species' middle temperature moved, so that no range is common."""
-    therm = open(CC.THERM).read()
+def mechanism(common, both_sides=False):
+    """The H2/air mechanism; common False: one species' middle temperature moved, so that no range is common; both_sides:
+    with two reactions more, whose catalyst stands on both sides (once with another coefficient)."""
+    therm, mech = open(CC.THERM).read(), open(CC.MECH).read()
+    if both_sides:
+        first = "H+O2=O+OH "
+        assert mech.count(first) == 1
+        mech = mech.replace(first, "O2+H2O=O+O+H2O 1.0E+15 -0.50 1.0E+05\nH+H2O=>H+H+OH 1.0E+10 0.30 3.0E+04\n" + first)
     if not common:
         line = next(l for l in therm.split("\n") if l.startswith("H2O2 ") and l.rstrip().endswith("1"))
         therm = therm.replace(line, line.replace("1000.00", " 999.00"))
-    return corefl.Chemistry(mech_text=open(CC.MECH).read(), therm_text=therm)
+    return corefl.Chemistry(mech_text=mech, therm_text=therm)
 
 
 @pytest.mark.parametrize("common", [True, False])
