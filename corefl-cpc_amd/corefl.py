@@ -291,12 +291,13 @@ class Solver:
         """Continue from a flowfield.plt of the same blocks (read_flowfield, Initialize.cu:97-345)."""
         self._ok(self._lib.corefl_read_flowfield(self._ctx, os.fsencode(path)))
 
-    KERNELS = ("viscous_flux", "viscous_exchange", "flux_x", "flux_y", "flux_z", "update", "boundary", "cfl_dt")
+    KERNELS = ("viscous_flux", "viscous_exchange", "flux_x", "flux_y", "flux_z", "update", "boundary", "cfl_dt",
+               "fluxes")
 
     def profile_kernels(self, reps=5):
         """Average ms per launch of each kernel class (HIP events on the context stream)."""
-        out = (ctypes.c_double * 8)()
-        self._ok(self._lib.corefl_profile_kernels(self._ctx, int(reps), out, 8))
+        out = (ctypes.c_double * len(self.KERNELS))()
+        self._ok(self._lib.corefl_profile_kernels(self._ctx, int(reps), out, len(self.KERNELS)))
         return dict(zip(self.KERNELS, list(out)))
 
     def get_int(self, name):

@@ -147,7 +147,8 @@ int corefl_read_flowfield(corefl_ctx *ctx, const char *path);
  * no tracing, src/gxl_lib/Time.cpp:4-20).  Runs `reps` launches of each kernel class of one stage on the
  * current state and writes the average milliseconds per launch into ms_out[0..n_out):
  *   0 viscous node fluxes, 1 viscous ghost exchange (all faces), 2 x flux, 3 y flux, 4 z flux,
- *   5 residual + RK update (rk = 1 coefficients), 6 boundary fills (all faces), 7 CFL step (local + reduce).
+ *   5 residual + RK update (rk = 1 coefficients), 6 boundary fills (all faces), 7 CFL step (local + reduce),
+ *   8 the fluxes of all directions in one launch, as a stage takes them (2 to 4 are the same kernel on one direction).
  * The state is advanced by the update launches; call it on a scratch context. */
 int corefl_profile_kernels(corefl_ctx *ctx, int reps, double *ms_out, int n_out);
 
