@@ -35,8 +35,8 @@ template<int NS> struct Cell {
 // source, and a last pass for the new temperature.  The stages are one loop around a single copy of the source, the
 // temperature iteration and the solve: written out, the kernel is 113 KB of code, more than the 64 KB instruction cache
 // of two CUs; rolled it is 57 KB.  An attempt of a wave takes 100 us, from 145 (2.1M igniting cells: 3.4 ms, from 4.9):
-// 21700 vector instructions (28600), 670 scalar loads (2060) and no vector loads of coefficients.  It is bound by its one
-// wave per SIMD: vector instructions are 37% of its cycles, scalar ones 24%, waits for scalar loads 27%.  Two waves at 256
+// 21700 vector instructions (28600), 680 scalar loads (2060) and no vector loads of coefficients.  It is bound by its one
+// wave per SIMD: vector instructions are 38% of its cycles, scalar ones 25%, waits for loads 27%.  Two waves at 256
 // registers keep 950 bytes a lane in scratch and take 4.9 ms.
 template<int NS>
 __device__ __forceinline__ void rok4e_attempt(const ChemMech *mp, Cell<NS> &s, double rtol, double atol) {
@@ -175,8 +175,8 @@ template<int NS> __device__ __forceinline__ void store_partial(const ChemBatch &
 // of the launch's lanes hold a cell.  An attempt of every cell takes 100 us here whatever their number up to one per
 // lane (65536 lanes), and in the cooperative kernel 60 us for every 8192 cells, so the lines cross near 13000 cells;
 // below, its shorter attempt counts.  When that is reached depends on how waves are scheduled; a cell's bits do not, since
-// both kernels round alike.  (200003 igniting cells, 5.6 attempts on average and 123 at most: 5.8 ms, 6.7 with
-// every cell handed over after its fourth attempt.)
+// both kernels round alike.  (200003 igniting cells, 19.8 attempts on average and 122 at most: 9.7 ms, 17.7 in this kernel
+// alone and 16.6 in the cooperative one.)
 template<int NS>
 __global__ __launch_bounds__(256) void k_chem_queue(const ChemMech *__restrict__ mp, ChemBatch b, double dt,
                                                     double rtol, double atol, int max_attempts, int *counter,

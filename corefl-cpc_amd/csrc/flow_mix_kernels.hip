@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256) void k_mix_viscous_node(DevBlock b, MixArrays 
   double e4[3] = {xx * Ex + xy * Ey + xz * Ez, ex * Ex + ey * Ey + ez * Ez, zx * Ex + zy * Ey + zz * Ez};
   const ChemMech &m = *x.mech;
   // before the gradients of the mass fractions: beside their 45 values, the coefficients that the lanes of a front read one by
-  // one cost the second wave per SIMD (306 registers instead of 212; 97^3 nodes XXX us instead of 799)
+  // one cost the second wave per SIMD (306 registers instead of 212; 97^3 nodes 440 us instead of 799)
   double h[NS], cp[NS];
   chemdev::h_cp<NS>(m, b.bv[id + 5 * sz], h, cp);
   double yk[NS], dk[NS], drv[NS][3];
@@ -749,8 +749,9 @@ __device__ __forceinline__ double mix_state(const ChemMech &m, double *q, double
 // cn: the frozen transport residual of Wu's splitting (update_cv_and_bv_rk_wu, StrangSplitting.cu:504-562:
 // the stage advances with R(U) - cn over dts * dt), or nullptr for the plain stage (dts = 1).
 // VISC: viscous order (0, 2, 8); SOURCE: with the explicit chemical source, which costs the stage its second wave per
-// SIMD (more than 256 registers against 218), so the stage without one is a kernel of its own.  It is bound by memory
-// (about 80 values read and 33 written per node); the tiles run along k first, so that the work-groups that share an
+// SIMD (more than 256 registers against 218), so the stage without one is a kernel of its own.  It is bound by the latency
+// of its loads (about 80 values read and 33 written per node): its two waves wait for memory 83% of their cycles at 2.02 GB
+// a launch, 2.9 TB/s, 55% of what a large copy reaches.  The tiles run along k first, so that the work-groups that share an
 // XCD's L2 at a time read each other's z fluxes: 1021 -> 691 us on 129^3 nodes, inviscid.
 template<bool RHS_ONLY, int VISC, bool SOURCE>
 __global__ __launch_bounds__(256) void k_mix_update(DevBlock b, MixArrays x, int rk, const double *__restrict__ dtp,

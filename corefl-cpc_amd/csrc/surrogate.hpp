@@ -1,5 +1,5 @@
 // Chemistry surrogate: a 12 -> 4x128 (GELU or hard swish) -> 10 MLP with BF16 weights and FP32 accumulation on the
-// gfx950 matrix cores.  Training (forward, backward, Adam) runs as tiled MFMA GEMMs with fused epilogues;
+// gfx950 matrix cores.  A training step is three kernels (32 rows through all layers and back, the weight gradients, Adam);
 // inference runs as one persistent kernel holding every weight in LDS, fused with the feature scaling, the
 // element-conserving projection, the temperature recovery and the fallback gate.
 #pragma once
@@ -130,7 +130,7 @@ struct SurrogateWork {
 
 // FP32 feature rows X [n][12] -> BF16 rows [n][16] (zero padded).
 hipError_t launch_rows_to_feat(const float *X, long n, unsigned short *feat, hipStream_t s);
-// Inference.  Raw mode: BF16 feature rows feat [n][16] (as launch_gather writes them) -> outputs y [n][10].
+// Inference.  Raw mode: BF16 feature rows feat [n][16] (as launch_rows_to_feat writes them) -> outputs y [n][10].
 hipError_t launch_mlp_raw(const MlpDev &net, long n, const unsigned short *feat, float *y, int blocks,
                           hipStream_t s);
 // Chemistry mode: every cell of b (n cells) is advanced by dt (b.dtc per cell if set) with the network

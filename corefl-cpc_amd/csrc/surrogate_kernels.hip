@@ -70,7 +70,7 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
 // A training step is three launches.  One layer's product on 8192 rows is 0.27 GFLOP, a quarter of a microsecond of
 // the matrix cores, so launches and memory round trips between layers were all of the time: as 32 launches with each
 // layer's activations, pre-activations and gradients through memory a step took 658 us (15 products at 33 us, the
-// column sums of the biases at 31 us, ten Adam launches).  Three kernels take 21 + 11 + 5 us, 47 us a step in a row:
+// column sums of the biases at 31 us, ten Adam launches).  Three kernels take 22 + 11 + 5 us, 39 us a step in a row:
 //   k_train_tile  32 rows through all layers and back: activations in LDS, pre-activations in registers
 //   k_train_grad  the weight gradients, which contract over all rows, in up to 16 (above 16384 rows 64) chunks
 //   k_train_adam  sums the chunks in order (no atomics: the same inputs give the same step) and updates everything
@@ -556,8 +556,8 @@ __device__ void chem_finish(const FusedArgs &a, long c, const float *o, bool in_
   }
   double t_new = t_net;
   if (ok) {
-    // chemdev::update_t with the coefficients read from LDS in every iteration (the same operations in the same
-    // order; the empty asm statement with a memory clobber keeps the compiler from hoisting those reads, which
+    // chemdev::update_t's iteration, to rounding, over the species' own fits with the coefficients read from LDS in every
+    // iteration (the empty asm statement with a memory clobber keeps the compiler from hoisting those reads, which
     // would hold every coefficient in registers)
     t_new = fmin(fmax(t_net, 200.0), 5000.0);
     double imw = 0;

@@ -127,7 +127,7 @@ def test_wu_splitting_step_matches_oracle(method, inv):
 
 def test_strang_tuned_launch_and_surrogate_fallback_agree():
     """A closed surrogate gate sends every cell through the exact fallback (the cooperative launch), and the
-    autotuned launch may be a one-lane one: the same operations distributed differently, equal to rounding."""
+    autotuned launch may be a one-lane one: the same operations distributed differently."""
     case = _case(4, 2, temporal=5, reaction=1)
     ref = None
     for mode in ("default", "tuned", "surrogate-closed"):
