@@ -68,7 +68,7 @@ def compare(case, mixture):
         assert np.max(np.abs(x - y)) <= 1e-13 * np.max(np.abs(y))
 
 
-@pytest.mark.parametrize("dims", [(6, 6, 6), (9, 7, 12), (10, 17, 9), (33, 12, 20)])
+@pytest.mark.parametrize("dims", [(6, 6, 6), (9, 7, 12), (10, 17, 9), (33, 12, 20), (20, 14, 1)])
 @pytest.mark.parametrize("recon,visc", [(5, 4), (4, 8), (4, 2), (4, 0)])
 def test_air_periodic_sides_at_once(dims, recon, visc):
     compare(ragged(cases.tgv(33, recon=recon, inviscid=3, visc=visc, cfl=0.2), dims), False)
