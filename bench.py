@@ -36,7 +36,7 @@ STEP_BYTES = 560.0
 # (40 B) written
 FLUX_BYTES = 112.0
 # flux kernel, per interface: FP64 operations (FMA counted twice) of WENO7-characteristic + AUSM+, as counted
-# by SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 on the 256^3 workload (42.3 GFLOP per launch over 257 x 257 x 258
+# by SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 on the 256^3 workload (126.8 GFLOP per launch over 3 x 257 x 257 x 258
 # interfaces; profiles/flow_tgv256_fp64_valu.md)
 FLUX_FLOP = 2480.0
 FP64_PEAK_TFLOPS = 78.6

@@ -3,8 +3,9 @@ objects in the built library (a compiler's choice that no value test sees)."""
 import os
 import struct
 
-import msgpack
 import pytest
+
+msgpack = pytest.importorskip("msgpack")
 
 LIB = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "corefl-cpc_amd", "libcorefl_amd.so")
 EM_AMDGPU, NT_AMDGPU_METADATA, PT_NOTE = 224, 32, 4
